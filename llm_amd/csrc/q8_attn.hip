@@ -328,259 +328,297 @@ extern "C" __global__ __launch_bounds__(512) void q8_attn_decode_w8(Q8_ATTN_PARA
 // Prefill attention: n query tokens at cache positions start .. start+n-1, each
 // seeing keys 0 .. its own position (causal), on v_mfma_f32_32x32x16_f16.
 //
-// Workgroup = (head, 32 queries), two waves splitting the 64-key tiles (wave w
-// takes tiles w, w+2, ...), combined through LDS at the end.  Per tile a wave
-// computes S^T = K Q^T (keys x queries) and O^T += V^T P^T (dims x queries),
-// so a lane always holds one query (lane % 32): its scores, its running max
-// and sum, and its output accumulators, and the softmax needs no transpose.
+// A workgroup is (head, 32 queries); its KS waves deal the 32-key tiles among
+// themselves (wave g takes tiles g, g + KS, ...) and combine their (max, sum,
+// output) through LDS at the end.  A wave's K and V tile go to its own 8 KB of
+// LDS by direct loads (16 bytes a lane, whole 128-byte rows): the next K is
+// loaded once the scores have read this one, the next V once the values have,
+// so each has half a tile's time to arrive and no wave waits for another.
+// Per tile a wave computes S^T = K Q^T (keys x queries) and O^T += V^T P^T
+// (dims x queries), so a lane always holds one query (lane % 32): its scores,
+// its running max and sum, and its output accumulators, and the softmax needs
+// no transpose; the V^T operand is read transposed (ds_read_b64_tr_b16).  Rows
+// of 128 bytes would put every row's 16-byte chunk c on the same banks, so row
+// k keeps its chunk c at c ^ (k % 8).
+//
 // f32 operands enter the MFMA exactly as two f16 parts (x = hi + lo, hi =
 // f16(x), lo = f16(x - hi), ~22 significant bits; products of f16 are exact
 // in f32): q for the scores, the probabilities for the values; keys and
 // values are the f16 cache itself.  Accumulation is f32.  Element k of an
 // MFMA operand sits in lane-half k / 8, slot k % 8, for A and B alike; D[m][n]
-// has n = lane % 32, m = 8(v/4) + 4(lane/32) + v%4.  Keys past the last
-// visible one read as zero values and -inf scores.  Heavier (later) query
-// tiles are launched first.
+// has n = lane % 32, m = 8(v/4) + 4(lane/32) + v%4.
+//
+// The softmax runs in base 2: q is multiplied by scale log2(e) with its power
+// of two taken out (Q8AttnPrefillArgs), before the split that rounds it to 22
+// bits anyway, so a weight is one fma and one v_exp_f32, with one rounding of
+// the exponent's argument.  A row's reference m moves only when its tile max
+// passes it by more than 8 (weights stay below 2^8, sums in f32), so the
+// accumulators are rescaled in few tiles; it starts finite, so that a row with
+// no visible key yet subtracts no infinity.
+// Heavier (later) query tiles of a head are launched first, and the workgroups
+// of a head run on one XCD (round-robin dispatch), whose L2 then serves the
+// head's cache rows to all of them.
+//
+// What bounds it: VALU and MFMA issue, about 1.55 us of a SIMD per 64 keys x
+// 32 queries at four waves a SIMD (32 MFMAs 0.54 us, 33 v_exp_f32 and some 200
+// other VALU the rest).  Against two waves a workgroup over 64-key tiles with
+// V transposed in registers and a nine-instruction exp per weight, 36 heads:
+// 512 tokens at 0 24.0 -> 13.8 us, 1000 at 3000 203 -> 96 us, 43 at 3000 72 ->
+// 20 us.  64-key tiles (twice the LDS, three waves a SIMD at most): 14.3, 105
+// and 20 us; two query tiles sharing a K/V tile in LDS: 15.0, 100 and 38 us.
 // ---------------------------------------------------------------------------
-#define Q8_ATTN_VT_STRIDE 72  /* f16 per V^T row in LDS: 64 keys + 8 of padding, 144 B (16-byte rows) */
+#define Q8_ATTN_KEYS 32                                /* keys of a tile */
+#define Q8_ATTN_TILE_BYTES (Q8_ATTN_KEYS * Q8_ATTN_HEAD_DIM * 2) /* of K, or of V */
+#define Q8_ATTN_O_PITCH 33                             /* f32 per dim row of a wave's outputs in LDS */
 
-// e^x for the softmax's x = s - max <= 0 (x = -inf or below the f32 range
-// gives 0): x = n ln2 + r with n = rint(x log2e) and r from a two-part ln2
-// (Cody-Waite reduction: ln2_hi has 15 significant bits, so n ln2_hi is exact
-// for |n| < 2^9), then e^r = 2^(r log2e) on v_exp_f32 (|r log2e| <= 1/2) and
-// 2^n by ldexp.  With a correctly rounded exp2 the result is within 0.85
-// ulp of e^x on [-87, 0] (checked in f32 emulation); v_exp_f32 adds its own
-// (at most 1 ulp).  Nine instructions where the library expf takes ~25.
-static __device__ __forceinline__ float exp_nonpos(float x) {
-    const float n = __builtin_rintf(x * 1.44269504f);
-    float r = __builtin_fmaf(-n, 0.693145751953125f, x);
-    r = __builtin_fmaf(-n, 1.42860682e-06f, r);
-    const float e = __builtin_ldexpf(__builtin_amdgcn_exp2f(r * 1.44269504f), (int)n);
-    return x >= -87.0f ? e : 0.0f;
-}
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) const uint8_t lds_bytes_t;
+typedef __attribute__((address_space(3))) void attn_lds_t;
 
+// x as f16 hi + lo, two values an instruction where there is one; the
+// remainder x - hi by one mixed-precision fma (exact), two values of hi a register.
 static __device__ __forceinline__ void split_f16(const float *x, f16x8 &hi, f16x8 &lo) {
+    union Parts {
+        unsigned w[4];
+        f16x8 v;
+    } hp, lp;
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const _Float16 h = (_Float16)x[i];
-        hi[i] = h;
-        lo[i] = (_Float16)(x[i] - (float)h);
+    for (int i = 0; i < 4; i++) {
+        hp.w[i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x[2 * i], x[2 * i + 1]}, f16x2));
+        float l0, l1;
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(l0) : "v"(hp.w[i]), "v"(x[2 * i]));
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=v"(l1)
+            : "v"(hp.w[i]), "v"(x[2 * i + 1]));
+        lp.w[i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){l0, l1}, f16x2));
     }
+    hi = hp.v;
+    lo = lp.v;
 }
 
-extern "C" __global__ __launch_bounds__(128) void q8_attn_prefill(Q8AttnPrefillArgs a) {
-    __shared__ __attribute__((aligned(16))) uint16_t vt_all[2][Q8_ATTN_HEAD_DIM * Q8_ATTN_VT_STRIDE];
-    __shared__ float xm[64], xl[64];
-    __shared__ __attribute__((aligned(16))) float xo[64][33];
+// The V^T operands of a 16-key step, dims 0-31 (v0) and 32-63 (v1): four
+// transposed reads of 4 keys x 16 dims each, in one block with their wait (as
+// builtins the compiler drains every direct load in flight before them, the
+// next tile's too).  OFF: the step's byte offset in the tile.
+template <int OFF>
+static __device__ __forceinline__ void read_vt(unsigned a0, unsigned a1, f16x8 &v0, f16x8 &v1) {
+    s16x4 p0, p1, p2, p3;
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
+        "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
+        "ds_read_b64_tr_b16 %3, %5 offset:%7\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(p0), "=&v"(p1), "=&v"(p2), "=&v"(p3)
+        : "v"(a0), "v"(a1), "i"(OFF), "i"(OFF + 8 * 128)
+        : "memory");
+    v0 = __builtin_bit_cast(f16x8, __builtin_shufflevector(p0, p1, 0, 1, 2, 3, 4, 5, 6, 7));
+    v1 = __builtin_bit_cast(f16x8, __builtin_shufflevector(p2, p3, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+
+template <int KS>
+static __device__ __forceinline__ void attn_prefill_body(const Q8AttnPrefillArgs &a) {
     constexpr int HD = Q8_ATTN_HEAD_DIM;
-    const int head = blockIdx.x / a.qtiles;
-    const int qt = a.qtiles - 1 - (blockIdx.x - head * a.qtiles);
+    constexpr int COMB = HD * Q8_ATTN_O_PITCH * 4;  // a wave's outputs, over the tiles' LDS
+    constexpr int PER_WAVE = COMB > 2 * Q8_ATTN_TILE_BYTES ? COMB : 2 * Q8_ATTN_TILE_BYTES;
+    constexpr int LOADS = Q8_ATTN_KEYS / 8;  // direct loads of a tile
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[KS * PER_WAVE];
+    __shared__ float xm[KS][32], xl[KS][32];
+    const int lane = threadIdx.x & 63;
+    const int kg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = lane >> 5;
+    const int r = lane & 31;
+    // grid workgroup -> (head, query tile), a contiguous run of items per XCD
+    const int total = a.n_head * a.qtiles;
+    const int xcd = blockIdx.x & 7;
+    const int item = xcd * (total >> 3) + min(xcd, total & 7) + (int)(blockIdx.x >> 3);
+    const int head = item / a.qtiles;
+    const int qt = a.qtiles - 1 - (item - head * a.qtiles);
     const int kvh = head / (a.n_head / a.n_kv);
     const int kv_dim = a.n_kv * HD;
     const int start = *a.position;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
-    const int h = lane >> 5;
-    const int r = lane & 31;
-    uint16_t *vt = vt_all[wave];
     const int qrow = qt * 32 + r;  // this lane's query
     const int qa = start + qrow;   // its cache position
     const bool qlive = qrow < a.n;
 
-    // Q^T operand, d-step s: q[qrow][16s + 8h .. +7] as f16 hi/lo
-    f16x8 qhi[4], qlo[4];
-    {
-        const float *src = a.q + ((size_t)min(qrow, a.n - 1) * a.n_head + head) * HD + 8 * h;
+    const int kend = min(start + min(qt * 32 + 32, a.n), a.capacity);  // keys [0, kend)
+    const int ntiles = (kend + Q8_ATTN_KEYS - 1) / Q8_ATTN_KEYS;
+    const int groups = min(KS, ntiles);  // waves that hold a tile
+
+    // Direct loads: load j of a tile brings rows 8j .. 8j+7, lane i row i / 8's
+    // chunk (i % 8) ^ (i / 8).
+    const int lrow = lane >> 3;
+    const int lchunk = ((lane & 7) ^ lrow) * 8;
+    const uint16_t *const khead = a.kcache + kvh * HD + lchunk;
+    const uint16_t *const vhead = a.vcache + kvh * HD + lchunk;
+    uint8_t *const kbuf = smem + kg * 2 * Q8_ATTN_TILE_BYTES;
+    uint8_t *const vbuf = kbuf + Q8_ATTN_TILE_BYTES;
+    auto load_tile = [&](const uint16_t *base, int t, uint8_t *dst) {
 #pragma unroll
-        for (int s = 0; s < 4; s++) {
-            f32x4 u0 = *(const f32x4 *)(src + 16 * s), u1 = *(const f32x4 *)(src + 16 * s + 4);
-            float x[8] = {u0[0], u0[1], u0[2], u0[3], u1[0], u1[1], u1[2], u1[3]};
-            if (!qlive)
-#pragma unroll
-                for (int i = 0; i < 8; i++) x[i] = 0.0f;
-            split_f16(x, qhi[s], qlo[s]);
-        }
-    }
-    float m = -INFINITY, l = 0.0f;
-    f32x16 o[2] = {};
-    const f32x16 zero16 = {};
-    const int last_q = min(qt * 32 + 31, a.n - 1);
-    const int kend = min(start + last_q + 1, a.capacity);  // keys [0, kend)
-    const int ntiles = (kend + 63) >> 6;
-    // K operand rows (keys p0 + 32kt + r), d-slices 16s + 8h, of this wave's
-    // tile t: the next tile's are loaded while the current one is computed
-    i32x4 kn[2][4];
-    auto load_k = [&](int t) {
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-            const int key = min(t * 64 + 32 * kt + r, a.capacity - 1);
-            const uint16_t *krow = a.kcache + (size_t)key * kv_dim + kvh * HD + 8 * h;
-#pragma unroll
-            for (int s = 0; s < 4; s++) kn[kt][s] = *(const i32x4 *)(krow + 16 * s);
+        for (int j = 0; j < LOADS; j++) {
+            const int key = min(t * Q8_ATTN_KEYS + 8 * j + lrow, kend - 1);  // rows past the last repeat it (masked)
+            __builtin_amdgcn_global_load_lds(base + (size_t)key * kv_dim, (attn_lds_t *)(dst + j * 1024), 16, 0, 0);
         }
     };
-    if (wave < ntiles) load_k(wave);
-    for (int t = wave; t < ntiles; t += 2) {
-        const int p0 = t * 64;
-        i32x4 kk[2][4];
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-            for (int s = 0; s < 4; s++) kk[kt][s] = kn[kt][s];
-        // S^T: keys x queries
-        f32x16 st[2];
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++) {
-            f32x16 acc = zero16;
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const f16x8 kv = __builtin_bit_cast(f16x8, kk[kt][s]);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qhi[s], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qlo[s], acc, 0, 0, 0);
-            }
-            st[kt] = acc;
-        }
-        // This tile's value rows (lane -> dims 2(lane%32), +1 at keys
-        // 16(lane/32) .. +15 and +32), then the next tile's keys; both land
-        // while the softmax runs.
-        const int dp = lane & 31;
-        unsigned w[2][16];
-#pragma unroll
-        for (int half_keys = 0; half_keys < 2; half_keys++) {
-            const int kb = 32 * half_keys + 16 * h;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                // keys past the last visible one: a clamped (in-bounds) load, then zero
-                const int key = p0 + kb + i;
-                const unsigned u = *(const unsigned *)(a.vcache + (size_t)min(key, kend - 1) * kv_dim + kvh * HD + 2 * dp);
-                w[half_keys][i] = key < kend ? u : 0u;
-            }
-        }
-        if (t + 2 < ntiles) load_k(t + 2);
-        // scale, causal mask, online softmax for query qrow; a tile whose last
-        // key precedes the workgroup's first query needs no mask
-        float tm = -INFINITY;
-        if (p0 + 63 <= start + qt * 32) {
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    st[kt][v] = st[kt][v] * a.scale;
-                    tm = fmaxf(tm, st[kt][v]);
-                }
-        } else {
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int p = p0 + 32 * kt + 8 * (v >> 2) + 4 * h + (v & 3);
-                    const float sc = (p <= qa) ? st[kt][v] * a.scale : -INFINITY;
-                    st[kt][v] = sc;
-                    tm = fmaxf(tm, sc);
-                }
-        }
-        tm = fmaxf(tm, __shfl_xor(tm, 32));
-        const float mn = fmaxf(m, tm);
-        // a wave's first tile may be all masked for its queries only if it is
-        // not tile 0; then m and mn stay -inf: no weight and no rescale
-        const float corr = (mn == -INFINITY) ? 1.0f : exp_nonpos(m - mn);
-        float rs = 0.0f;
-#pragma unroll
-        for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const float e = (mn == -INFINITY) ? 0.0f : exp_nonpos(st[kt][v] - mn);
-                st[kt][v] = e;
-                rs += e;
-            }
-        rs += __shfl_xor(rs, 32);
-        l = l * corr + rs;
-        m = mn;
-#pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) o[dt][v] *= corr;
-        // V^T tile (wave-private) from the value rows
-#pragma unroll
-        for (int half_keys = 0; half_keys < 2; half_keys++) {
-            const int kb = 32 * half_keys + 16 * h;
-            i32x4 r0[2], r1[2];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                r0[j >> 2][j & 3] =
-                    (int)__builtin_amdgcn_perm(w[half_keys][2 * j + 1], w[half_keys][2 * j], 0x05040100u);
-                r1[j >> 2][j & 3] =
-                    (int)__builtin_amdgcn_perm(w[half_keys][2 * j + 1], w[half_keys][2 * j], 0x07060302u);
-            }
-            i32x4 *d0 = (i32x4 *)(vt + (2 * dp) * Q8_ATTN_VT_STRIDE + kb);
-            i32x4 *d1 = (i32x4 *)(vt + (2 * dp + 1) * Q8_ATTN_VT_STRIDE + kb);
-            d0[0] = r0[0];
-            d0[1] = r0[1];
-            d1[0] = r1[0];
-            d1[1] = r1[1];
-        }
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's V^T stores are done
+    // the wave's direct loads have landed: all of them, or all but the last tile half's
+    auto landed = [&](bool all) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (all)
+            __builtin_amdgcn_s_waitcnt(Q8_VMCNT_IMM(0));
+        else
+            __builtin_amdgcn_s_waitcnt(Q8_VMCNT_IMM(LOADS));
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_wave_barrier();
-        // O^T += V^T P^T over four 16-key steps
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // the wave's LDS reads have returned: the buffer may be loaded again
+    auto reads_done = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    float m = -1e30f, l = 0.0f;  // l: this lane's half of the keys
+    f32x16 o[2] = {};
+    if (kg < groups) {
+        // q's loads first (they need no position), then the first tile's
+        f32x4 qv[8];
+        {
+            const float *src = a.q + ((size_t)min(qrow, a.n - 1) * a.n_head + head) * HD + 8 * h;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+            for (int s = 0; s < 8; s++) qv[s] = *(const f32x4 *)(src + 16 * (s >> 1) + 4 * (s & 1));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load_tile(khead, kg, kbuf);
+        load_tile(vhead, kg, vbuf);
+        // Q^T operand, d-step s: q[qrow][16s + 8h .. +7] as f16 hi/lo
+        f16x8 qhi[4], qlo[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            float x[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[i] = qlive ? qv[2 * s + (i >> 2)][i & 3] * a.q_mult : 0.0f;
+            split_f16(x, qhi[s], qlo[s]);
+        }
+        const float s2 = a.s_mult;
+        const int lim = min(qa, kend - 1);  // last key this lane's query sees
+        int koff[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) koff[s] = r * 128 + (((2 * s + h) ^ (r & 7)) << 4);
+        // V^T: 16 lanes read 4 keys x 16 dims; lane i the 8 bytes of key i / 4, dims 4 (i % 4)
+        unsigned voff[2];
+        {
+            const int i = lane & 15, key = 4 * h + (i >> 2);
+#pragma unroll
+            for (int dt = 0; dt < 2; dt++)
+                voff[dt] = (unsigned)(uintptr_t)(lds_bytes_t *)vbuf + key * 128 +
+                           (((4 * dt + 2 * ((lane >> 4) & 1) + ((i >> 1) & 1)) ^ key) << 4) + 8 * (i & 1);
+        }
+        f32x16 st;
+        // O^T += V^T P^T over the 16 keys from 16 J
+        auto values = [&](auto jc) {
+            constexpr int J = decltype(jc)::value;
+            // slots 0-3: keys 16J + 4h + ..; slots 4-7: keys 16J + 8 + 4h + ..
             float pv[8];
 #pragma unroll
-            for (int i = 0; i < 8; i++) pv[i] = st[j >> 1][8 * (j & 1) + i];
-            f16x8 phi, plo;
+            for (int i = 0; i < 8; i++) pv[i] = st[8 * J + i];
+            f16x8 phi, plo, v0, v1;
             split_f16(pv, phi, plo);
+            read_vt<J * 16 * 128>(voff[0], voff[1], v0, v1);
+            o[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v0, phi, o[0], 0, 0, 0);
+            o[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v1, phi, o[1], 0, 0, 0);
+            o[0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v0, plo, o[0], 0, 0, 0);
+            o[1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v1, plo, o[1], 0, 0, 0);
+        };
+        for (int t = kg; t < ntiles; t += KS) {
+            const bool next = t + KS < ntiles;
+            landed(false);  // K (V may still be in flight)
+            st = (f32x16){};
 #pragma unroll
-            for (int dt = 0; dt < 2; dt++) {
-                const uint16_t *row = vt + (32 * dt + r) * Q8_ATTN_VT_STRIDE + 16 * j + 4 * h;
-                const uint2 lo4 = *(const uint2 *)row;
-                const uint2 hi4 = *(const uint2 *)(row + 8);
-                const i32x4 va = {(int)lo4.x, (int)lo4.y, (int)hi4.x, (int)hi4.y};
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, va), phi, o[dt], 0, 0, 0);
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, va), plo, o[dt], 0, 0, 0);
+            for (int s = 0; s < 4; s++) {  // S^T: keys x queries
+                const f16x8 kv = *(const f16x8 *)(kbuf + koff[s]);
+                st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qhi[s], st, 0, 0, 0);
+                st = __builtin_amdgcn_mfma_f32_32x32x16_f16(kv, qlo[s], st, 0, 0, 0);
             }
+            reads_done();
+            if (next) load_tile(khead, t + KS, kbuf);
+            // a tile whose last key precedes the tile's first query needs no mask
+            const int p0 = t * Q8_ATTN_KEYS;
+            if (p0 + Q8_ATTN_KEYS - 1 > min(start + qt * 32, kend - 1)) {
+#pragma unroll
+                for (int v = 0; v < 16; v++) st[v] = p0 + 8 * (v >> 2) + 4 * h + (v & 3) <= lim ? st[v] : -INFINITY;
+            }
+            float top[2] = {st[0], st[1]};
+#pragma unroll
+            for (int v = 2; v < 16; v++) top[v & 1] = fmaxf(top[v & 1], st[v]);
+            const float tm = xor_max<32>(fmaxf(top[0], top[1])) * s2;
+            if (__ballot(tm > m + 8.0f)) {
+                const float mn = fmaxf(m, tm);
+                const float corr = __builtin_amdgcn_exp2f(m - mn);
+                m = mn;
+                l *= corr;
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    o[0][v] *= corr;
+                    o[1][v] *= corr;
+                }
+            }
+            float rs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                st[v] = __builtin_amdgcn_exp2f(__builtin_fmaf(st[v], s2, -m));
+                rs[v & 3] += st[v];
+            }
+            l += (rs[0] + rs[1]) + (rs[2] + rs[3]);
+            landed(!next);  // V (the next K may still be in flight)
+            values(std::integral_constant<int, 0>{});
+            values(std::integral_constant<int, 1>{});
+            reads_done();
+            if (next) load_tile(vhead, t + KS, vbuf);
         }
-        __builtin_amdgcn_s_waitcnt(0xc07f);  // the tile's V^T reads are done before the next tile overwrites it
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __builtin_amdgcn_wave_barrier();
     }
-    // combine the two waves' partial softmax states (wave 1 -> LDS -> wave 0)
-    if (wave == 1) {
-        if (h == 0) {
-            xm[r] = m;
-            xl[r] = l;
-        }
+
+    // Combine the waves' softmax states through LDS; the first two waves
+    // finish one half of the dims each.
+    float *const comb = reinterpret_cast<float *>(smem);
+    __syncthreads();  // the tiles are read
+    if (kg < groups) {
+        const float lt = xor_add<32>(l);
+        float *dst = comb + kg * HD * Q8_ATTN_O_PITCH;
 #pragma unroll
         for (int dt = 0; dt < 2; dt++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) xo[32 * dt + 8 * (v >> 2) + 4 * h + (v & 3)][r] = o[dt][v];
+            for (int v = 0; v < 16; v++) dst[(32 * dt + 8 * (v >> 2) + 4 * h + (v & 3)) * Q8_ATTN_O_PITCH + r] = o[dt][v];
+        if (h == 0) {
+            xm[kg][r] = m;
+            xl[kg][r] = lt;
+        }
     }
     __syncthreads();
-    if (wave == 1) return;
-    const float m1 = xm[r], l1 = xl[r];
-    const float mt = fmaxf(m, m1);  // finite: key 0 is in tile 0 (wave 0) and visible to every query
-    const float c0 = expf(m - mt);
-    const float c1 = (m1 == -INFINITY) ? 0.0f : expf(m1 - mt);
-    const float lt = l * c0 + l1 * c1;
-    // res[dt][4g + e]: dim 32 dt + 8 g + 4 h + e of this lane's query (0 for
-    // the padding queries of the last tile)
-    float res[2][16];
+    static_assert(KS >= 2, "two waves finish the dims");
+    if (kg > 1) return;
+    const int dt = kg;
+    float mt = xm[0][r];
+    for (int k = 1; k < groups; k++) mt = fmaxf(mt, xm[k][r]);
+    // res[4g + e]: dim 32 dt + 8 g + 4 h + e of this lane's query (0 for the
+    // padding queries of the last tile)
+    float res[16], lt = 0.0f;
 #pragma unroll
-    for (int dt = 0; dt < 2; dt++)
+    for (int v = 0; v < 16; v++) res[v] = 0.0f;
+    for (int k = 0; k < groups; k++) {
+        const float c = __builtin_amdgcn_exp2f(xm[k][r] - mt);
+        lt = __builtin_fmaf(xl[k][r], c, lt);
+        const float *src = comb + (k * HD + 32 * dt + 4 * h) * Q8_ATTN_O_PITCH + r;
 #pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int d = 32 * dt + 8 * (v >> 2) + 4 * h + (v & 3);
-            res[dt][v] = qlive ? (o[dt][v] * c0 + xo[d][r] * c1) / lt : 0.0f;
-        }
+        for (int v = 0; v < 16; v++) res[v] = __builtin_fmaf(src[(8 * (v >> 2) + (v & 3)) * Q8_ATTN_O_PITCH], c, res[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < 16; v++) res[v] = qlive ? res[v] / lt : 0.0f;
     if (a.out && qlive) {
-        float *orow = a.out + ((size_t)qrow * a.n_head + head) * HD;
+        float *orow = a.out + ((size_t)qrow * a.n_head + head) * HD + 32 * dt + 4 * h;
 #pragma unroll
-        for (int dt = 0; dt < 2; dt++)
-#pragma unroll
-            for (int g = 0; g < 4; g++)
-                *(f32x4 *)(orow + 32 * dt + 8 * g + 4 * h) =
-                    (f32x4){res[dt][4 * g], res[dt][4 * g + 1], res[dt][4 * g + 2], res[dt][4 * g + 3]};
+        for (int g = 0; g < 4; g++)
+            *(f32x4 *)(orow + 8 * g) = (f32x4){res[4 * g], res[4 * g + 1], res[4 * g + 2], res[4 * g + 3]};
     }
     if (a.xq) {
         // The head's 64 dims are Q8_0 blocks 2 head and 2 head + 1 of the
@@ -590,25 +628,28 @@ extern "C" __global__ __launch_bounds__(128) void q8_attn_prefill(Q8AttnPrefillA
         // the pair (r, r + 32) trades two values per chunk, then quantizes
         // as q8_quantize does (quant_store, the block peak across the pair).
         const int nb = 2 * a.n_head;
+        float e[4][4];
 #pragma unroll
-        for (int dt = 0; dt < 2; dt++) {
-            float e[4][4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const float v0 = res[dt][4 * c], v1 = res[dt][4 * c + 1];
-                const float v2 = res[dt][4 * c + 2], v3 = res[dt][4 * c + 3];
-                const float p0 = __shfl_xor(v0, 32), p1 = __shfl_xor(v1, 32);
-                const float p2 = __shfl_xor(v2, 32), p3 = __shfl_xor(v3, 32);
-                e[0][c] = h == 0 ? v0 : p2;  // 8c + 0 | 8c + 2
-                e[1][c] = h == 0 ? p0 : v2;  // 8c + 4 | 8c + 6
-                e[2][c] = h == 0 ? v1 : p3;  // 8c + 1 | 8c + 3
-                e[3][c] = h == 0 ? p1 : v3;  // 8c + 5 | 8c + 7
-            }
-            float peak = half_peak(e);
-            peak = fmaxf(peak, __shfl_xor(peak, 32));
-            quant_store(e, peak, a.xq, a.xs, (size_t)qt * nb + 2 * head + dt, 32 * h + r, h == 0, a.f16);
+        for (int c = 0; c < 4; c++) {
+            const float v0 = res[4 * c], v1 = res[4 * c + 1];
+            const float v2 = res[4 * c + 2], v3 = res[4 * c + 3];
+            const float p0 = __shfl_xor(v0, 32), p1 = __shfl_xor(v1, 32);
+            const float p2 = __shfl_xor(v2, 32), p3 = __shfl_xor(v3, 32);
+            e[0][c] = h == 0 ? v0 : p2;  // 8c + 0 | 8c + 2
+            e[1][c] = h == 0 ? p0 : v2;  // 8c + 4 | 8c + 6
+            e[2][c] = h == 0 ? v1 : p3;  // 8c + 1 | 8c + 3
+            e[3][c] = h == 0 ? p1 : v3;  // 8c + 5 | 8c + 7
         }
+        const float peak = xor_max<32>(half_peak(e));
+        quant_store(e, peak, a.xq, a.xs, (size_t)qt * nb + 2 * head + dt, 32 * h + r, h == 0, a.f16);
     }
+}
+
+// Four waves a workgroup (four workgroups a CU), or eight where there are too
+// few workgroups to fill the chip with four (run_attn_prefill).
+extern "C" __global__ __launch_bounds__(256, 4) void q8_attn_prefill(Q8AttnPrefillArgs a) { attn_prefill_body<4>(a); }
+extern "C" __global__ __launch_bounds__(512, 4) void q8_attn_prefill_k8(Q8AttnPrefillArgs a) {
+    attn_prefill_body<8>(a);
 }
 
 // ---------------------------------------------------------------------------

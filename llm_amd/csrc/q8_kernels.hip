@@ -21,6 +21,8 @@
 //                                                              (gpu.cu rmsnorm_rows, rmsnorm_quantize_rows 351-407)
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "q8_layout.h"
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));

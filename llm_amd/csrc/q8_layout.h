@@ -297,7 +297,6 @@ typedef struct {
  * as the reference's device cache (gpu.cu kv_append 506-519). */
 #define Q8_ATTN_HEAD_DIM 64 /* the head width the attention kernels are built for */
 #define Q8_ATTN_COMBINE_MAX 8 /* most attention splits a GEMV prologue combines */
-#define Q8_ATTN_TILE 64     /* prefill: queries and keys per tile */
 
 typedef struct {
     float *q;            /* [n][n_head][head_dim] f32, rotated in place */
@@ -331,7 +330,7 @@ typedef struct {
     float *out;             /* [n][n_head][head_dim], or null */
     const int *position;    /* device: cache position of query 0 */
     int n, n_head, n_kv, capacity, qtiles;
-    float scale;
+    float q_mult, s_mult;   /* scale log2(e) = q_mult s_mult: q_mult in [1/2, 1) (or +-0), s_mult a power of two */
     uint8_t *xq;            /* non-null: the output also as prepared Q8_0 (units, as q8_quantize writes them) */
     float *xs;              /* its block scales */
     int f16;                /* 1: f16 prepared units */

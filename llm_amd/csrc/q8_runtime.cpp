@@ -98,6 +98,7 @@ enum Fn {
     F_GEMV_HG8_3_E0, F_GEMV_HG16_3_E0, F_GEMV_HG16_6_E0, F_GEMV_HS8_3_E0, F_GEMV_HS16_6_E0,
     F_GEMV_HP16_3, F_GEMV_HP16_6, F_GEMV_HP16_3_E0, F_GEMV_HP16_6_E0,
     F_ATTN_DECODE_W8,
+    F_ATTN_PREFILL_K8,
     F_COUNT
 };
 
@@ -137,6 +138,7 @@ const char *const kFnNames[F_COUNT] = {
     "q8_gemv_hg8_l3_e0", "q8_gemv_hg16_l3_e0", "q8_gemv_hg16_l6_e0", "q8_gemv_hs8_l3_e0", "q8_gemv_hs16_l6_e0",
     "q8_gemv_hp16_l3", "q8_gemv_hp16_l6", "q8_gemv_hp16_l3_e0", "q8_gemv_hp16_l6_e0",
     "q8_attn_decode_w8",
+    "q8_attn_prefill_k8",
 };
 
 // Every kernel of the code object with its metadata (q8_manifest.h, from the
@@ -2565,7 +2567,9 @@ int run_attn_prefill(q8_ctx *c, const float *q, q8_dptr kcache, q8_dptr vcache, 
     a.n_kv = n_kv;
     a.capacity = capacity;
     a.qtiles = (int)ceil_div(n, 32);
-    a.scale = scale;
+    int e2 = 0;
+    a.q_mult = (float)std::frexp((double)scale * 1.4426950408889634, &e2);
+    a.s_mult = (float)std::ldexp(1.0, e2);
     if (p) {
         const int k = n_head * Q8_ATTN_HEAD_DIM;
         const int nb = k / 32;
@@ -2582,7 +2586,9 @@ int run_attn_prefill(q8_ctx *c, const float *q, q8_dptr kcache, q8_dptr vcache, 
         p->k = k;
         p->format = fmt;
     }
-    return launch(c, F_ATTN_PREFILL, (unsigned)(n_head * a.qtiles), 128, 0, &a, sizeof a);
+    const unsigned wgs = (unsigned)(n_head * a.qtiles);
+    if (wgs > (unsigned)c->cu_count) return launch(c, F_ATTN_PREFILL, wgs, 256, 0, &a, sizeof a);
+    return launch(c, F_ATTN_PREFILL_K8, wgs, 512, 0, &a, sizeof a);
 }
 
 int check_attention(q8_ctx *c, q8_dptr qp, q8_dptr kcache, q8_dptr vcache, q8_dptr position, int n, int n_head,
