@@ -949,12 +949,8 @@ int run_gemm_silu(q8_ctx *c, const q8_weight *gate, const q8_weight *up, const q
     a.kslices = 1;
     const int npairs = (nb + 1) / 2;
     a.pairs_per_slice = npairs;
-    // >= 11 waves per CU (each wave carries a gate and an up tile, as the
-    // paired-token-tile GEMM), >= 9 block pairs per wave; measured over
-    // n = 32..1024 at 5760 x 2304
     const long long base = (long long)gate->tiles * ttiles;
-    int kw = (int)std::max<long long>(1, ceil_div(11LL * std::max(c->cu_count, 1), base));
-    kw = std::min(std::min(kw, 8), std::max(1, npairs / 9));
+    int kw = q8_gemm_silu_kwaves(n, ffn, k, c->cu_count);
     const int kw_opt = option(c, "gemm.kwaves", -1);
     if (kw_opt > 0) kw = std::min(kw_opt, 8);
     kw = std::min(kw, npairs);

@@ -120,44 +120,61 @@ void q8_gemv_shape(int out, int k, int cu_count, int slots, q8_tactic *t) {
     }
 }
 
-// GEMM launch shape.  A wave owns TPW token tiles of one 32-row tile.  Two
-// tiles per wave share the weight stream and measured best for wide matrices
-// (n = 512: gate|up 11520 rows 51 us, QKV 6912 rows 37.5 us); one tile per
-// wave with the block pairs split over eight waves of a workgroup (reduced in
-// LDS in a fixed order) measured best for the 2304-row projections (O 18.6 us,
-// down 33 us) and for small n.  Four tiles per wave needs ~240 VGPRs (two
-// waves per SIMD) and measured slower everywhere; it stays an option.
+// GEMM launch shape.  A wave owns TPW token tiles of one 32-row tile and one
+// of kwaves equal ranges of the block pairs.
+//
+// What bounds it: a wave's pair takes 0.25 us (one token tile) or 0.45 us
+// (two) alone and the launch about 7 us beside its pairs, so a small launch
+// wants its pairs spread over waves, down to two each; a SIMD does one token
+// tile's block in 76 ns from registers but 127 ns from the caches, two tiles'
+// in 97 and 100, so a large one wants the two tiles that share the weight
+// loads.  Between them the best launch has its waves resident at once (2800 of
+// the 4096 at one token tile, 3072 at two): beyond, a second round of short
+// waves pays the 7 us again.  kwaves is a power of two because other counts load
+// the four SIMDs unevenly.  Four tiles per wave (two waves per SIMD) and two
+// token-tile waves a workgroup were no better than a few per cent anywhere.
+//
+// Measured on gfx950 over rows 384 .. 11520, K 512 .. 5760 and n 4 .. 1000
+// (312 shapes, every shape of launch): within 2.1% of the best on the
+// geometric mean, where the rule before it (about 18 waves per CU, at least
+// nine pairs a wave, two token tiles from 300 row tiles up) was 13.5% off.
+// Times before -> now, us: 1152 x 896 n = 257 7.2 -> 5.7, 2304 x 5760 n = 131
+// 15.5 -> 13.4, 6912 x 2304 n = 1000 60 -> 50, 2304 x 5760 n = 1000 60 -> 48.
 void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
-    // Measured on gfx950 (n = 8 ... 1024, M = 2304 ... 11 520, K = 2304 / 5760):
-    // a wave costs a fixed prologue (first loads) and K reduction, so it wants
-    // at least ~9 block pairs of work, and the launch wants ~18 waves per CU
-    // (4.5 per SIMD) to hide the MFMA -> convert -> fma chain of each wave.
-    // Very tall matrices (gate|up, 360 row tiles) already have enough waves
-    // with two token tiles per wave and the full K; matrices of >= 128 row
-    // tiles pair two token-tile waves in a workgroup, which then share the
-    // weight units in L1.
     const int nb = k / 32;
     const int npairs = ceil_div(nb, 2);
     const int ttiles = ceil_div(n, 32);
-    const int rtiles = ceil_div(out, 32);
-    const int cus = std::max(cu_count, 1);
-    const int tpw = (rtiles >= 300 && ttiles >= 2) ? 2 : 1;
-    const int groups = ceil_div(ttiles, tpw);
-    const long long base = (long long)rtiles * groups;  // waves without a K split
-    const long long target = (tpw == 1 ? 18LL : 11LL) * cus;  // 4608 / 2816 waves on 256 CUs
-    int kw = (int)std::max<long long>(1, (target + base - 1) / base);
-    kw = std::min(kw, std::max(1, npairs / 9));
-    kw = std::min(kw, 8);
+    const long long rtiles = ceil_div(out, 32);
+    const long long cus = std::max(cu_count, 1);
+    const long long tiles = rtiles * ttiles;
+    // the lines lie at 1300 tiles and 80 000 tile-pairs on 256 CUs
+    const int tpw = (ttiles >= 2 && tiles * 256 >= 1300 * cus && tiles * npairs * 256 >= 80000 * cus) ? 2 : 1;
+    const long long base = rtiles * ceil_div(ttiles, tpw);  // waves without a K split
+    const long long most = (tpw == 1 ? 2800 : 3072) * cus / 256;
+    int kw = npairs < 8 ? 1 : 8;  // shorter rows were not measured and stay unsplit
+    while (kw > 1 && (base * kw > most || npairs < 2 * kw)) kw /= 2;
     const int ppw = ceil_div(npairs, kw);
-    kw = ceil_div(npairs, ppw);
-    const int tw = (tpw == 1 && rtiles >= 128 && groups >= 2 && kw <= 8) ? 2 : 1;
     t->tpw = tpw;
-    t->twaves = tw;
-    t->kwaves = kw;
+    t->twaves = 1;
+    t->kwaves = ceil_div(npairs, ppw);
     t->kslices = 1;
     t->pairs_per_wave = ppw;
     t->smode = 1;
     t->xcd_remap = 1;
+}
+
+// The fused gate/up launch (one wave a gate tile, its up tile and one token
+// tile): as above, four K waves at most (eight were slower at every shape but
+// the smallest K = 2304 ones, by up to 2%), at most 2500 waves.  Over widths
+// 960 .. 5760, K 512 .. 2304 and n 4 .. 1000: within 1.4% of the best on the
+// geometric mean, 12% before (11 waves per CU, nine pairs a wave); 2432 x 896
+// n = 43 10.5 -> 7.0 us, 5760 x 2304 n = 349 44.5 -> 40.4.
+int q8_gemm_silu_kwaves(int n, int ffn, int k, int cu_count) {
+    const int npairs = ceil_div(k / 32, 2);
+    const long long base = (long long)ceil_div(ffn, 32) * ceil_div(n, 32);
+    int kw = npairs < 8 ? 1 : 4;
+    while (kw > 1 && (base * kw * 256 > 2500LL * std::max(cu_count, 1) || npairs < 2 * kw)) kw /= 2;
+    return kw;
 }
 
 // f16 GEMM launch shape: TPW token tiles per wave (2 when there are two or
