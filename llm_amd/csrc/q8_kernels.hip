@@ -1051,6 +1051,11 @@ static __device__ __forceinline__ void gemv_rs_body(const RsHot &hot, const Q8Ge
         qv[i] = q8_weight_load(qbase + (size_t)b * qstride);
         dd[i] = (unsigned)sbase[(size_t)b * Q8_TILE_ROWS];
     }
+    // the residual with them: after the row sums it would be a dependent load
+    // at the end of the launch
+    const int row = tile * Q8_TILE_ROWS + srow;
+    float res = 0.0f;
+    if (mbias) res = mbias[min(row, mrows - 1)];
     __builtin_amdgcn_sched_barrier(0);
 
     // zero each row's tail up to a multiple of four blocks (chain_row reads
@@ -1122,8 +1127,7 @@ static __device__ __forceinline__ void gemv_rs_body(const RsHot &hot, const Q8Ge
         acc = vbuf[r];
         for (int w2 = 1; w2 < nw; w2++) acc = acc + vbuf[w2 * RS + r];
     }
-    const int row = tile * Q8_TILE_ROWS + srow;
-    if (row < mrows) my[row] = mbias ? acc + mbias[row] : acc;
+    if (row < mrows) my[row] = mbias ? acc + res : acc;
 }
 
 #define Q8_RS_PARAMS                                                                                  \
@@ -1501,6 +1505,34 @@ static __device__ __forceinline__ void gemv_rsg_body(const RsgHot &hot, const Q8
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (HOT) select_member();  // the epilogue's member, read while the weights stream in
     const int tile = SILU ? gtile : gtile - mtb;  // within the member
+    // the tail wave's rotation, formed while the weights stream in: at the end
+    // of the launch the frequency would be a dependent load with the sine and
+    // cosine behind it (scalar loads: a vector load's wait would be for the
+    // weights issued before it, too)
+    const int row = tile * Q8_TILE_ROWS + srow;
+    const bool in_cache = rope_position >= 0 && rope_position < a.capacity;
+    bool rot = false;
+    float sn = 0.0f, cs = 1.0f;
+    if (!SILU && rope_pos && wave == 0 && mi < 2 && in_cache && a.n_rot > 0) {
+        typedef __attribute__((address_space(4))) const float scalar_f32;
+        const scalar_f32 *freqs = (const scalar_f32 *)(uintptr_t)a.rope_freq;
+        int d = (tile * Q8_TILE_ROWS + slice * RS) % a.head_dim;  // dim of the slice's first row
+        float fv[RS / 2];  // of its row pairs
+        int dp = 0;        // the lane's pair's first dim
+#pragma unroll
+        for (int i = 0; i < RS / 2; i++) {
+            fv[i] = freqs[min(d >> 1, (a.n_rot >> 1) - 1)];
+            dp = r >> 1 == i ? d : dp;
+            d = d + 2 == a.head_dim ? 0 : d + 2;
+        }
+#pragma unroll
+        for (int i = 0; i < RS / 2; i++) asm volatile("" : "+s"(fv[i]));  // all loaded at once
+        float freq = 0.0f;
+#pragma unroll
+        for (int i = 0; i < RS / 2; i++) freq = r >> 1 == i ? fv[i] : freq;
+        rot = dp < a.n_rot;
+        sincosf((float)rope_position * freq, &sn, &cs);
+    }
     __shared__ double npart[4];
     if (norm && threadIdx.x < 256) {
         double ss = 0.0;
@@ -1592,26 +1624,18 @@ static __device__ __forceinline__ void gemv_rsg_body(const RsgHot &hot, const Q8
         sums[0] *= s;
         sums[1] *= s;
     }
-    const int row = tile * Q8_TILE_ROWS + srow;
     if constexpr (SILU) {
         if (row < mrows) my[row] = silu_f32(sums[0]) * sums[1];
     } else if (rope_pos) {
         // gemv_body's RoPE + KV append: rows 2i and 2i+1 of a head are lanes
         // r and r ^ 1 of wave 0 (RS is even, slices start at even rows)
-        const float other = __shfl_xor(sums[0], 1);
-        const int pos = rope_position;
-        const bool in_cache = pos >= 0 && pos < a.capacity;
+        const float other = xor_partner<1>(sums[0]);
         if (row < mrows) {
-            const int d = row % a.head_dim;
-            const int pair = d >> 1;
-            const bool even = (d & 1) == 0;
+            const bool even = (row & 1) == 0;  // head_dim is even
             const float x0 = even ? sums[0] : other;
             const float x1 = even ? other : sums[0];
             float y0 = x0, y1 = x1;
-            if (in_cache && mi < 2 && 2 * pair < a.n_rot) {
-                const float angle = (float)pos * a.rope_freq[pair];
-                float sn, cs;
-                sincosf(angle, &sn, &cs);
+            if (rot) {
                 y0 = x0 * cs - x1 * sn;
                 y1 = x0 * sn + x1 * cs;
             }
@@ -1620,7 +1644,7 @@ static __device__ __forceinline__ void gemv_rsg_body(const RsgHot &hot, const Q8
                 my[row] = out;
             } else if (in_cache) {
                 uint16_t *cache = mi == 1 ? a.kcache : a.vcache;
-                cache[(size_t)pos * mrows + row] = (uint16_t)f16_bits(out);
+                cache[(size_t)rope_position * mrows + row] = (uint16_t)f16_bits(out);
             }
         }
     } else if (row < mrows) {
