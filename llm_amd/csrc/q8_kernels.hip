@@ -1975,42 +1975,72 @@ extern "C" __global__ __launch_bounds__(256) void q8_quantize(Q8QuantArgs a) {
 // its half of the rotated pair -- the angle (position * freq), sincosf and
 // the f16 narrowing of that kernel.  q is written rotated in f32; k rotated
 // and v as they are go only to the f16 caches, at row position + token.
+//
+// The angles' sines and cosines depend on (token, pair) alone.  Where the
+// launch has LDS for them (`table`: [TPW][32 tokens][16 pairs] (sin, cos),
+// filled by fill_rope_table), they were formed by all of a tile's waves while
+// its first operands were on the way; otherwise here, where the pair's two
+// lanes compute eight of their 16 each and swap.
+// ---------------------------------------------------------------------------
+static __device__ __forceinline__ int rope_pair(const Q8GemmArgs &a, int row) { return (row % a.head_dim) >> 1; }
+
+// A wave's share (part of parts) of the table of TPW token tiles; `pair` and
+// `freq` are those of local pair lane % 16.
+template <int TPW>
+static __device__ __forceinline__ void fill_rope_table(const Q8GemmArgs &a, int pair, float freq, int tt0, f32x2 *table,
+                                                       int part, int parts, int lane) {
+    const int start = *a.rope_pos;
+    for (int i = part * 64 + lane; i < TPW * 512; i += parts * 64) {  // [TPW][32 tokens][16 pairs]
+        float sn = 0.0f, cs = 1.0f;
+        if (2 * pair < a.n_rot) sincosf((float)(start + tt0 * Q8_TILE_TOKENS + (i >> 4)) * freq, &sn, &cs);
+        table[i] = (f32x2){sn, cs};
+    }
+}
+
 template <int TPW>
 static __device__ __forceinline__ void store_rope_tiles(const Q8GemmArgs &a, const Q8GemmMember &mem, int mi,
-                                                        const f32x16 (&acc)[TPW], int tt0, int o, int h) {
+                                                        const f32x16 (&acc)[TPW], int tt0, int o, int h,
+                                                        const f32x2 *table) {
     const int start = *a.rope_pos;
-    const int d = o % a.head_dim;
-    const int pair = d >> 1;
-    const bool even = (d & 1) == 0;
+    const int pair = rope_pair(a, o);
+    const bool even = (o & 1) == 0;  // head_dim is even
     const bool rot = mi < 2 && 2 * pair < a.n_rot;
-    const float freq = rot ? a.rope_freq[pair] : 0.0f;
     uint16_t *cache = mi == 1 ? a.kcache : a.vcache;
     const int odd = even ? 0 : 1;  // of the pair's lanes r, r ^ 1, the odd one takes elements 8..15
 #pragma unroll
     for (int t = 0; t < TPW; t++) {
         if (tt0 + t >= a.ttiles) continue;  // wave-uniform
         const int tok0 = (tt0 + t) * Q8_TILE_TOKENS + 4 * h;  // token of element i: tok0 + 8(i/4) + i%4
-        // The pair's two lanes need the same 16 angles: each computes eight
-        // (the even lane elements 0-7, the odd lane 8-15) and they swap.
         float sn[16], cs[16];
         if (mi < 2) {  // wave-uniform
+            if (table) {
+                const f32x2 *tp = table + t * 512 + 4 * h * 16 + ((o & 31) >> 1);
 #pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int i = j + 8 * odd;
-                const float angle = (float)(start + tok0 + 8 * (i >> 2) + (i & 3)) * freq;
-                float sj, cj;
-                sincosf(angle, &sj, &cj);
-                const float so = __shfl_xor(sj, 1), co = __shfl_xor(cj, 1);
-                sn[j] = odd ? so : sj;
-                cs[j] = odd ? co : cj;
-                sn[j + 8] = odd ? sj : so;
-                cs[j + 8] = odd ? cj : co;
+                for (int i = 0; i < 16; i++) {
+                    const f32x2 v = tp[(8 * (i >> 2) + (i & 3)) * 16];
+                    sn[i] = v.x;
+                    cs[i] = v.y;
+                }
+            } else {
+                const float freq = rot ? a.rope_freq[pair] : 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int i = j + 8 * odd;
+                    const float angle = (float)(start + tok0 + 8 * (i >> 2) + (i & 3)) * freq;
+                    float sj, cj;
+                    sincosf(angle, &sj, &cj);
+                    const float so = xor_partner<1>(sj), co = xor_partner<1>(cj);
+                    sn[j] = odd ? so : sj;
+                    cs[j] = odd ? co : cj;
+                    sn[j + 8] = odd ? sj : so;
+                    cs[j + 8] = odd ? cj : co;
+                }
             }
         }
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const float x = acc[t][i];
-            const float other = __shfl_xor(x, 1);  // the partner row, same token
+            const float other = xor_partner<1>(x);  // the partner row, same token
             const int tok = tok0 + 8 * (i >> 2) + (i & 3);
             const int pos = start + tok;
             const bool in_cache = pos >= 0 && pos < a.capacity;
@@ -2035,9 +2065,10 @@ static __device__ __forceinline__ void store_rope_tiles(const Q8GemmArgs &a, con
 
 template <int TPW>
 static __device__ __forceinline__ void store_tiles(const Q8GemmArgs &a, const Q8GemmMember &mem, int mi,
-                                                   const f32x16 (&acc)[TPW], int tt0, int o, int h) {
+                                                   const f32x16 (&acc)[TPW], int tt0, int o, int h,
+                                                   const f32x2 *rope_table = nullptr) {
     if (a.rope_pos) {
-        store_rope_tiles<TPW>(a, mem, mi, acc, tt0, o, h);
+        store_rope_tiles<TPW>(a, mem, mi, acc, tt0, o, h, rope_table);
         return;
     }
     if (o >= mem.rows) return;
@@ -2285,12 +2316,28 @@ static __device__ __forceinline__ void gemm_body(const Q8GemmArgs &a) {
         }
     };
 
+    const int KW = (blockDim.x >> 6) / TW;
+    // a q or k tile's rotations, in the time its first operands take
+    f32x2 *const rope_table = reinterpret_cast<f32x2 *>(gsm + (size_t)(KW - 1) * TW * TPW * 1024) + tw * TPW * 512;
+    // (the frequency's load goes out ahead of them, so its wait is not theirs)
+    const bool rope = a.rope_pos && mi < 2;
+    const int rpair = rope ? rope_pair(a, g * Q8_TILE_ROWS + 2 * (lane & 15)) : 0;
+    float rfreq = 0.0f;
+    if (rope && a.n_rot > 0) rfreq = a.rope_freq[min(rpair, (a.n_rot >> 1) - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    auto rope_fill = [&]() {
+        if (rope) fill_rope_table<TPW>(a, rpair, rfreq, tt0, rope_table, kw, KW, lane);
+    };
+
     // Full pairs, two per iteration with ping-pong operand sets (no register
     // copies); each set's loads are issued one pair ahead of its use, and
     // sched_barrier keeps the compiler from sinking them next to their use.
+    if (p_begin >= full_end) rope_fill();
     if (p_begin < full_end) {
         GemmOps<TPW> qa, qb;
         load_full(qa, 2 * p_begin);
+        __builtin_amdgcn_sched_barrier(0);
+        rope_fill();
         int p = p_begin;
         for (; p + 1 < full_end; p += 2) {
             load_full(qb, 2 * (p + 1));
@@ -2316,7 +2363,6 @@ static __device__ __forceinline__ void gemm_body(const Q8GemmArgs &a) {
         for (int t = 0; t < TPW; t++) step(q, t, 2 * full_end, false);
     }
 
-    const int KW = (blockDim.x >> 6) / TW;
     if (KW > 1) {
         // reduce the K-split waves in a fixed order: kw = 0 adds 1, 2, ...
         if (kw > 0) {
@@ -2381,7 +2427,7 @@ static __device__ __forceinline__ void gemm_body(const Q8GemmArgs &a) {
     }
     if (kw != 0) return;
 
-    store_tiles<TPW>(a, mem, mi, acc, tt0, g * Q8_TILE_ROWS + r, h);
+    store_tiles<TPW>(a, mem, mi, acc, tt0, g * Q8_TILE_ROWS + r, h, rope_table);
 }
 
 // ---------------------------------------------------------------------------

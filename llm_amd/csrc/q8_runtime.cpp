@@ -1016,6 +1016,8 @@ int run_gemm(q8_ctx *c, const Member *m, int count, const q8_prepared *p, int n,
         rows_total += m[i].w->out;
     }
     q8_tactic t = plan(c, n, rows_total, k, 1, Q8_PREPARED_I8);
+    if (rope && t.smode && !t.pipe && option(c, "gemm.tpw", 0) <= 0 && option(c, "gemm.twaves", 0) <= 0)
+        q8_gemm_rope_shape(n, rows_total, &t);
     if (no_split && t.kslices > 1) {
         t.kslices = 1;
         t.pairs_per_wave = (int)ceil_div((nb + 1) / 2, std::max(1, t.kwaves));
@@ -1050,7 +1052,9 @@ int run_gemm(q8_ctx *c, const Member *m, int count, const q8_prepared *p, int n,
     const bool pipe = t.pipe && t.smode && a.kslices == 1 && tpw <= 2;
     const int max_threads = (tpw == 1 && !pipe) ? 1024 : 512;
     if (threads > max_threads) return fail(Q8_ERR_UNSUPPORTED, "gemm: %d threads per workgroup", threads);
-    const unsigned lds = (unsigned)((kwaves - 1) * a.twaves * tpw * 64 * 16 * sizeof(float));
+    // the K reduction, and a q, k, v group's table of rotations (fill_rope_table)
+    const unsigned lds = (unsigned)((kwaves - 1) * a.twaves * tpw * 64 * 16 * sizeof(float) +
+                                    (rope ? (size_t)a.twaves * tpw * 16 * 32 * 2 * sizeof(float) : 0));
     Fn f = pipe ? (tpw == 2 ? F_GEMM_P_T2 : F_GEMM_P_T1)
                 : !t.smode ? F_GEMM_S0_T1 : tpw == 4 ? F_GEMM_S1_T4 : tpw == 2 ? F_GEMM_S1_T2 : F_GEMM_S1_T1;
     // one token tile: every weight byte is read by one wave, once (option

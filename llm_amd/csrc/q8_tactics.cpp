@@ -163,6 +163,17 @@ void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
     t->xcd_remap = 1;
 }
 
+// A q, k, v group with its rotation in the epilogue: the plain group's K split
+// (the results are its bits), one token tile a wave.  The epilogue is long and a
+// wave of two token tiles runs it twice in a row (6912 x 2304: n = 512 34.0 us
+// against 32.1, n = 1000 59.5 against 53.4).  From 128 row tiles up two token-tile
+// waves share a workgroup and its weight loads where the token tiles pair off (in
+// a layer at n = 43 0.6 us less; 3 us more where one wave idles, n = 257).
+void q8_gemm_rope_shape(int n, int out, q8_tactic *t) {
+    t->tpw = 1;
+    t->twaves = (ceil_div(out, 32) >= 128 && ceil_div(n, 32) % 2 == 0) ? 2 : 1;
+}
+
 // The fused gate/up launch (one wave a gate tile, its up tile and one token
 // tile): as above, four K waves at most (eight were slower at every shape but
 // the smallest K = 2304 ones, by up to 2%), at most 2500 waves.  Over widths
