@@ -168,10 +168,11 @@ void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
 // wave of two token tiles runs it twice in a row (6912 x 2304: n = 512 34.0 us
 // against 32.1, n = 1000 59.5 against 53.4).  From 128 row tiles up two token-tile
 // waves share a workgroup and its weight loads where the token tiles pair off (in
-// a layer at n = 43 0.6 us less; 3 us more where one wave idles, n = 257).
+// a layer at n = 43 0.6 us less; 3 us more where one wave idles, n = 257), up to
+// the workgroup's 16 waves (the rule splits K over eight at most, an option over more).
 void q8_gemm_rope_shape(int n, int out, q8_tactic *t) {
     t->tpw = 1;
-    t->twaves = (ceil_div(out, 32) >= 128 && ceil_div(n, 32) % 2 == 0) ? 2 : 1;
+    t->twaves = (ceil_div(out, 32) >= 128 && ceil_div(n, 32) % 2 == 0 && t->kwaves <= 8) ? 2 : 1;
 }
 
 // The fused gate/up launch (one wave a gate tile, its up tile and one token
