@@ -153,9 +153,26 @@ static __device__ __forceinline__ void attn_decode_body(const AttnHead &hd, cons
     float *const part_acc_ = hd.part_acc;
     float *const part_ms_ = hd.part_acc + (size_t)n_head_ * splits_ * Q8_ATTN_HEAD_DIM;
     const int position = *hd.position;
-    const int head = blockIdx.x / splits_;
-    const int split = blockIdx.x - head * splits_;
-    const int kvh = head / (n_head_ / n_kv_);
+    // Workgroup -> (head, split).  The heads of a kv head read the same rows:
+    // (kv head, split, head of the group), a contiguous run of them per XCD
+    // (round-robin dispatch), leaves all but the first of a group their rows in
+    // that XCD's L2: dealt over all eight, every XCD fetched the group's rows.
+    // Four decode layers of 32 heads on 8: 129 -> 119 us at 3500 positions, 116
+    // -> 110 at 1500; two heads a group or 300 positions: within 0.5%.  With a
+    // kv head of its own a head shares nothing.
+    const int gsize = n_head_ / n_kv_;
+    int head = blockIdx.x / splits_;
+    int split = blockIdx.x - head * splits_;
+    int kvh = head;
+    if (gsize > 1) {
+        const int total = n_head_ * splits_;
+        const int xcd = blockIdx.x & 7;
+        const int item = xcd * (total >> 3) + min(xcd, total & 7) + (int)(blockIdx.x >> 3);
+        const int pair = item / gsize;
+        kvh = pair / splits_;
+        split = pair - kvh * splits_;
+        head = kvh * gsize + item - pair * gsize;
+    }
     const int kv_dim = n_kv_ * HD;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
