@@ -307,6 +307,19 @@ static __device__ __forceinline__ double xor_add_f64(double v) {
         return v + __hiloint2double((int)__float_as_uint(phi), (int)__float_as_uint(plo));
     }
 }
+// The butterfly over a wave, on DPP and lane swaps (a step of __shfl_xor on a
+// double is an LDS permute of each half and their wait).  In the norms' rows,
+// whose launch is one chain of latencies: two layers at n = 43 122.0 -> 121.2 us,
+// a small model's at n = 257 108.2 -> 106.8 us, four norms each.
+static __device__ __forceinline__ double wave_sum_f64(double v) {
+    v = xor_add_f64<32>(v);
+    v = xor_add_f64<16>(v);
+    v = xor_add_f64<8>(v);
+    v = xor_add_f64<4>(v);
+    v = xor_add_f64<2>(v);
+    return xor_add_f64<1>(v);
+}
+
 // The folded RMSNorm's scale from q8_rmsnorm_row's four wave sums:
 // 1 / sqrt(mean square + eps), the mean square rounded once from f64.
 static __device__ __forceinline__ float norm_scale(const double *npart, int k, float eps) {
@@ -662,12 +675,7 @@ static __device__ __forceinline__ void gemv_body(const Q8GemvArgs &a) {
                 for (int e = 0; e < 4; e++) ss += (double)(nx[j][e] * nx[j][e]);
             }
         }
-        ss = xor_add_f64<32>(ss);
-        ss = xor_add_f64<16>(ss);
-        ss = xor_add_f64<8>(ss);
-        ss = xor_add_f64<4>(ss);
-        ss = xor_add_f64<2>(ss);
-        ss = xor_add_f64<1>(ss);
+        ss = wave_sum_f64(ss);
         if (lane == 0) npart[wave] = ss;
     }
     float nscale = 1.0f;
@@ -1543,12 +1551,7 @@ static __device__ __forceinline__ void gemv_rsg_body(const RsgHot &hot, const Q8
                 for (int e = 0; e < 4; e++) ss += (double)(nx[jj][e] * nx[jj][e]);
             }
         }
-        ss = xor_add_f64<32>(ss);
-        ss = xor_add_f64<16>(ss);
-        ss = xor_add_f64<8>(ss);
-        ss = xor_add_f64<4>(ss);
-        ss = xor_add_f64<2>(ss);
-        ss = xor_add_f64<1>(ss);
+        ss = wave_sum_f64(ss);
         if (lane == 0) npart[wave] = ss;
     }
     if (norm) {
@@ -1751,12 +1754,7 @@ static __device__ __forceinline__ void gemv_rsp_body(const RsgHot &hot, const Q8
                 for (int e = 0; e < 4; e++) ss += (double)(nx[jj][e] * nx[jj][e]);
             }
         }
-        ss = xor_add_f64<32>(ss);
-        ss = xor_add_f64<16>(ss);
-        ss = xor_add_f64<8>(ss);
-        ss = xor_add_f64<4>(ss);
-        ss = xor_add_f64<2>(ss);
-        ss = xor_add_f64<1>(ss);
+        ss = wave_sum_f64(ss);
         if (lane == 0) npart[wave] = ss;
     }
     if (norm) {
@@ -3224,8 +3222,7 @@ extern "C" __global__ __launch_bounds__(256) void q8_rmsnorm(Q8NormArgs a) {
         ss += (double)(v2 * v2);
         ss += (double)(v3 * v3);
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+    ss = wave_sum_f64(ss);
     const float mean_square = (float)(ss / (double)k);
     const float scale = 1.0f / sqrtf(mean_square + a.eps);
 
@@ -3256,7 +3253,7 @@ extern "C" __global__ __launch_bounds__(256) void q8_rmsnorm(Q8NormArgs a) {
                 e[3][c] = live ? x11 : 0.0f;  // J[h][3] = 5 + 2h
             }
             float peak = half_peak(e);
-            peak = fmaxf(peak, __shfl_xor(peak, 1));
+            peak = xor_max<1>(peak);
             if (b0 + (lane >> 1) < nb)
                 quant_store(e, peak, a.xq, a.xs, (size_t)tt * nb + b, 32 * h + (t & 31), h == 0, a.f16);
         }
@@ -3319,8 +3316,7 @@ extern "C" __global__ __launch_bounds__(256) void q8_rmsnorm_row(Q8NormArgs a) {
             for (int e = 0; e < 4; e++) ss += (double)(xv[j][e] * xv[j][e]);
         }
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off);
+    ss = wave_sum_f64(ss);
     if ((tid & 63) == 0) part[tid >> 6] = ss;
     __syncthreads();
     const double total = (part[0] + part[1]) + (part[2] + part[3]);
@@ -3372,7 +3368,7 @@ extern "C" __global__ __launch_bounds__(256) void q8_rmsnorm_row(Q8NormArgs a) {
                 e[3][c] = hi.y;  // J[h][3] = 5 + 2h
             }
             float peak = half_peak(e);
-            peak = fmaxf(peak, __shfl_xor(peak, 1));
+            peak = xor_max<1>(peak);
             if (128 * g + (tid >> 1) < nb)
                 quant_store(e, peak, a.xq, a.xs, (size_t)tt * nb + b, 32 * h + (t & 31), h == 0, a.f16);
         }
