@@ -2145,6 +2145,17 @@ static __device__ __forceinline__ void gemm_rider(const Q8GemmArgs &a, int rider
     }
 }
 
+// Item of workgroup b of nwg where every XCD (round-robin dispatch) takes a
+// contiguous run of the items, for any nwg: a run is one longer on the first
+// nwg % 8 XCDs.  With runs only where eight divides nwg, the other launches'
+// token groups read their row tile's weights into every L2: 9402 x 1024
+// n = 202 17.3 -> 13.4 us, on the geometric mean over such launches 6% at 2 to 14
+// tiles a CU, 3% over all and for gate/up.
+static __device__ __forceinline__ int xcd_item(int nwg, int b) {
+    const int xcd = b & 7;
+    return xcd * (nwg >> 3) + min(xcd, nwg & 7) + (b >> 3);
+}
+
 // The compute workgroup of grid workgroup `b`, or -1 for a cache rider (which
 // it has then run).
 static __device__ __forceinline__ int gemm_workgroup(const Q8GemmArgs &a, int b) {
@@ -2156,11 +2167,7 @@ static __device__ __forceinline__ int gemm_workgroup(const Q8GemmArgs &a, int b)
         }
         if (a.rider_first) b -= a.riders;
     }
-    if (a.xcd_remap) {
-        const int per = a.nwg >> 3;
-        b = (b & 7) * per + (b >> 3);
-    }
-    return b;
+    return a.xcd_remap ? xcd_item(a.nwg, b) : b;
 }
 
 template <int TPW>
@@ -2654,11 +2661,7 @@ static __device__ __forceinline__ void gemm_h_body(const Q8GemmArgs &a) {
     const int KW = (blockDim.x >> 6) / RW;
     const int rw = wave % RW;
     const int kw = wave / RW;
-    int wg = blockIdx.x;
-    if (a.xcd_remap) {
-        const int per = a.nwg >> 3;
-        wg = (wg & 7) * per + (wg >> 3);
-    }
+    const int wg = a.xcd_remap ? xcd_item(a.nwg, blockIdx.x) : (int)blockIdx.x;
     const int rg = wg / a.tgroups;
     const int tg = wg - rg * a.tgroups;
     const int rt = rg * RW + rw;                       // global row tile (may be past the end)
@@ -2908,11 +2911,7 @@ static __device__ __forceinline__ void gemm_p_body(const Q8GemmArgs &a) {
     const int TW = a.twaves;
     const int tw = wave % TW;
     const int kw = wave / TW;
-    int wg = blockIdx.x;
-    if (a.xcd_remap) {
-        const int per = a.nwg >> 3;
-        wg = (wg & 7) * per + (wg >> 3);
-    }
+    const int wg = a.xcd_remap ? xcd_item(a.nwg, blockIdx.x) : (int)blockIdx.x;
     const int rt = wg / a.tgroups;
     const int tg = wg - rt * a.tgroups;
     const int tt0 = (tg * TW + tw) * TPW;

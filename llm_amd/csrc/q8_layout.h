@@ -219,7 +219,7 @@ typedef struct {
     int twaves;     /* waves along the tokens per workgroup (each TPW token tiles) */
     int tgroups;    /* ceil(ttiles / (twaves * TPW)) */
     int nwg;        /* workgroups launched (total_rtiles * tgroups * kslices) */
-    int xcd_remap;  /* 1: map workgroups so one row tile's token groups share an XCD */
+    int xcd_remap;  /* 1: a contiguous run of workgroups per XCD, so one row tile's token groups share one */
     int kslices;          /* S: workgroups splitting the block pairs of one output tile group */
     int pairs_per_slice;  /* ceil(ceil(nb/2) / S) */
     int pairs_per_wave;   /* ceil(pairs_per_slice / kwaves) */

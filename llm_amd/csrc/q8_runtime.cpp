@@ -960,7 +960,7 @@ int run_gemm_silu(q8_ctx *c, const q8_weight *gate, const q8_weight *up, const q
     const long long nwg = base;
     if (nwg > 0x7fffffffLL - 4096) return fail(Q8_ERR_UNSUPPORTED, "gemm_silu: grid of %lld workgroups", nwg);
     a.nwg = (int)nwg;
-    a.xcd_remap = nwg % 8 == 0 ? 1 : 0;
+    a.xcd_remap = 1;
     a.oq = static_cast<uint8_t *>(c->act2_ws);
     a.os = reinterpret_cast<float *>(static_cast<uint8_t *>(c->act2_ws) + align_up(qbytes, kAlign));
     a.of16 = fmt == Q8_PREPARED_F16 ? 1 : 0;
@@ -1047,7 +1047,7 @@ int run_gemm(q8_ctx *c, const Member *m, int count, const q8_prepared *p, int n,
     const long long nwg = groups * a.kslices;
     if (nwg > 0x7fffffffLL - 4096) return fail(Q8_ERR_UNSUPPORTED, "gemm: grid of %lld workgroups", nwg);
     a.nwg = (int)nwg;
-    a.xcd_remap = (t.xcd_remap && nwg % 8 == 0) ? 1 : 0;
+    a.xcd_remap = t.xcd_remap ? 1 : 0;
     const int threads = 64 * a.twaves * kwaves;
     const bool pipe = t.pipe && t.smode && a.kslices == 1 && tpw <= 2;
     const int max_threads = (tpw == 1 && !pipe) ? 1024 : 512;
@@ -1113,7 +1113,7 @@ int run_gemm_h(q8_ctx *c, const Member *m, int count, const q8_prepared *p, int 
     const long long nwg = ceil_div(rt, rw) * (long long)a.tgroups;
     if (nwg > 0x7fffffffLL) return fail(Q8_ERR_UNSUPPORTED, "gemm_h: grid of %lld workgroups", nwg);
     a.nwg = (int)nwg;
-    a.xcd_remap = (t.xcd_remap && nwg % 8 == 0) ? 1 : 0;
+    a.xcd_remap = t.xcd_remap ? 1 : 0;
     const size_t stage =
         (size_t)kw * Q8_GEMM_H_STAGES * (i8 ? Q8_GEMM_L_BUF_BYTES(tpw, rw) : Q8_GEMM_H_BUF_BYTES(tpw, rw));
     const size_t reduce = (size_t)(kw - 1) * rw * tpw * 64 * 16 * sizeof(float);

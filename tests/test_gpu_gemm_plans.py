@@ -59,6 +59,33 @@ def test_gemm_on_both_sides_of_the_lines(gpu, n, rows, k, tpw, kwaves):
         gpu.release(w)
 
 
+# workgroup counts on both sides of a multiple of the eight XCDs, and below it
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 15, 41])
+@pytest.mark.parametrize("option", [None, "gemm.pipe", "gemm.lds", "gemm.f16"])
+def test_every_tile_has_its_workgroup(gpu, option, tiles):
+    n, rows, k = 20, 32 * tiles, 544
+    r = np.random.default_rng(SEED + tiles)
+    w = q8.Weight(oracle.make_q8_weight(r, rows, k), k, rows)
+    x = oracle.make_activations(r, n, k, outlier_rate=0.01)
+    xb, yb = gpu.alloc(4 * n * k), gpu.alloc(4 * n * rows)
+    xb.upload(x)
+    yb.upload(np.full(n * rows, np.nan, np.float32))
+    try:
+        print(f"\n{option} {tiles} row tiles", flush=True)
+        if option:
+            gpu.set_option(option, 1)
+        gpu.matmul(w, xb, 0, n, yb, 0)
+        got = yb.download(np.float32, n * rows).reshape(n, rows)
+        assert_parity(got, oracle.matmul(w.data, k, rows, x, n), exact_at(w.data, k, rows, x, n),
+                      f"{option} n={n} rows={rows} k={k}")
+    finally:
+        if option:
+            gpu.set_option(option, -1)
+        xb.free()
+        yb.free()
+        gpu.release(w)
+
+
 @pytest.mark.parametrize("n,heads,kv,n_rot,e,position,kwaves", [(*c, -1) for c in [
     (2, 4, 2, 64, 256, 0), (32, 22, 11, 64, 1536, 5),       # one token tile
     (33, 24, 24, 64, 1536, 9), (64, 32, 16, 64, 1536, 0),   # 144 and 128 row tiles, paired: 1024 threads
