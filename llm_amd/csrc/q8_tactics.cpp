@@ -121,7 +121,8 @@ void q8_gemv_shape(int out, int k, int cu_count, int slots, q8_tactic *t) {
 }
 
 // GEMM launch shape.  A wave owns TPW token tiles of one 32-row tile and one
-// of kwaves equal ranges of the block pairs.
+// of kwaves equal ranges of the block pairs; a workgroup holds the kwaves of one
+// such tile, or of two neighbouring ones (twaves).
 //
 // What bounds it: a wave's pair takes 0.25 us (one token tile) or 0.45 us
 // (two) alone and the launch about 7 us beside its pairs, so a small launch
@@ -131,15 +132,25 @@ void q8_gemv_shape(int out, int k, int cu_count, int slots, q8_tactic *t) {
 // loads.  Between them the best launch has its waves resident at once (2800 of
 // the 4096 at one token tile, 3072 at two): beyond, a second round of short
 // waves pays the 7 us again.  kwaves is a power of two because other counts load
-// the four SIMDs unevenly.  Four tiles per wave (two waves per SIMD) and two
-// token-tile waves a workgroup were no better than a few per cent anywhere.
+// the four SIMDs unevenly, and eight only while every workgroup has a CU to
+// itself: a second one of eight waves doubles that CU's time (4608 x 2304 n = 64
+// 9.4 us with eight, 8.6 with four).  From four to five workgroups a CU two waves
+// each leave a SIMD with one more than the others, so rows of 32 pairs and more
+// split over four there (3072 x 2304 n = 384 14.8 -> 13.9).  With two or four token
+// tiles and one to two workgroups a CU, two neighbouring tiles share a workgroup
+// and its weight loads in L1 (5760 x 2304 n = 64 9.4 -> 9.0, 4096 x 4096 n = 100 12.8 ->
+// 12.0); where it leaves CUs idle it is 10 to 40% slower, and with more token
+// tiles slower beside the riders of a layer (2304 x 5760 n = 192 by 1.8).  Four
+// tiles per wave (two waves per SIMD) was never better.
 //
-// Measured on gfx950 over rows 384 .. 11520, K 512 .. 5760 and n 4 .. 1000
-// (312 shapes, every shape of launch): within 2.1% of the best on the
-// geometric mean, where the rule before it (about 18 waves per CU, at least
-// nine pairs a wave, two token tiles from 300 row tiles up) was 13.5% off.
-// Times before -> now, us: 1152 x 896 n = 257 7.2 -> 5.7, 2304 x 5760 n = 131
-// 15.5 -> 13.4, 6912 x 2304 n = 1000 60 -> 50, 2304 x 5760 n = 1000 60 -> 48.
+// The lines are fit to gfx950 times over rows 200 .. 12000, K 512 .. 8192 and n
+// 2 .. 1024, every shape of launch: 1120 calls with cold weights, 1.9% slower than
+// the best on the geometric mean, and each projection of 119 decoder layers with
+// their riders, 4.4%.  Eight waves up to 350 tiles, no paired tiles and two token
+// tiles a wave from 1300 tiles and 80 000 tile-pairs gave 2.5% and 5.3%; about 18
+// waves per CU with at least nine pairs a wave 14%.  Times of the three (the last
+// first), us: 1152 x 896 n = 257 7.2, 5.7, 5.7; 5760 x 2304 n = 64 9.0, 9.4, 9.0;
+// 2304 x 5760 n = 131 15.5, 13.4, 13.4; n = 1000 52.7, 47.6, 47.6.
 void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
     const int nb = k / 32;
     const int npairs = ceil_div(nb, 2);
@@ -147,16 +158,19 @@ void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
     const long long rtiles = ceil_div(out, 32);
     const long long cus = std::max(cu_count, 1);
     const long long tiles = rtiles * ttiles;
-    // the lines lie at 1300 tiles and 80 000 tile-pairs on 256 CUs
-    const int tpw = (ttiles >= 2 && tiles * 256 >= 1300 * cus && tiles * npairs * 256 >= 80000 * cus) ? 2 : 1;
-    const long long base = rtiles * ceil_div(ttiles, tpw);  // waves without a K split
+    // the lines lie at 870 tiles and 64 000 tile-pairs on 256 CUs
+    const int tpw = (ttiles >= 2 && tiles * 256 >= 870 * cus && tiles * npairs * 256 >= 64000 * cus) ? 2 : 1;
+    const long long groups = ceil_div(ttiles, tpw);
+    const long long base = rtiles * groups;  // waves without a K split
     const long long most = (tpw == 1 ? 2800 : 3072) * cus / 256;
-    int kw = npairs < 8 ? 1 : 8;  // shorter rows were not measured and stay unsplit
-    while (kw > 1 && (base * kw > most || npairs < 2 * kw)) kw /= 2;
+    const bool four = tpw == 1 && npairs >= 32 && base > 4 * cus && base <= 5 * cus;
+    int kw = npairs < 8 ? 1 : tpw == 1 && base <= cus ? 8 : 4;  // rows below eight pairs were not measured and stay unsplit
+    while (kw > 1 && ((base * kw > most && !(four && kw == 4)) || npairs < 2 * kw)) kw /= 2;
     const int ppw = ceil_div(npairs, kw);
+    kw = ceil_div(npairs, ppw);
     t->tpw = tpw;
-    t->twaves = 1;
-    t->kwaves = ceil_div(npairs, ppw);
+    t->twaves = (groups == 2 || groups == 4) && kw >= 2 && kw <= 4 && base > cus && base <= 2 * cus ? 2 : 1;
+    t->kwaves = kw;
     t->kslices = 1;
     t->pairs_per_wave = ppw;
     t->smode = 1;

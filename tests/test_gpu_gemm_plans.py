@@ -31,9 +31,11 @@ def gpu():
 PLANS = [
     (64, 100, 448, 1, 1), (33, 100, 480, 1, 4),                 # seven pairs: unsplit; eight: two each
     (5, 2304, 1024, 1, 8), (32, 1300, 544, 1, 3),               # two each over eight waves; nine pairs in three
-    (97, 2720, 2304, 1, 8), (129, 2304, 5760, 1, 4),            # 340 tiles: all resident at eight; 360: at four
-    (480, 2624, 4096, 1, 2), (512, 2624, 4096, 2, 4),           # 1230 and 1312 tiles
-    (512, 2624, 3872, 2, 4), (512, 2624, 3840, 1, 2),           # 80 032 and 78 720 tile-pairs
+    (97, 2048, 2304, 1, 8), (97, 2720, 2304, 1, 4),             # 256 tiles: a CU each, eight waves; 340: token tiles paired
+    (64, 4128, 2304, 1, 4), (129, 2304, 5760, 1, 4),            # 258 tiles, paired; 360 in five: unpaired
+    (480, 2624, 3328, 1, 4), (480, 2624, 4096, 2, 4),           # 63 960 and 78 720 tile-pairs
+    (512, 2624, 4096, 2, 4), (512, 2624, 3872, 2, 4),
+    (512, 2624, 3840, 2, 4), (256, 4000, 4736, 2, 4),           # paired: two token tiles in each of two waves
     (489, 5000, 2080, 2, 2), (1000, 6912, 1088, 2, 1),          # a half-empty last token tile; no K split
 ]
 
