@@ -1017,7 +1017,7 @@ int run_gemm(q8_ctx *c, const Member *m, int count, const q8_prepared *p, int n,
     }
     q8_tactic t = plan(c, n, rows_total, k, 1, Q8_PREPARED_I8);
     if (rope && t.smode && !t.pipe && option(c, "gemm.tpw", 0) <= 0 && option(c, "gemm.twaves", 0) <= 0)
-        q8_gemm_rope_shape(n, rows_total, &t);
+        q8_gemm_rope_shape(n, rows_total, k, c->cu_count, &t);
     if (no_split && t.kslices > 1) {
         t.kslices = 1;
         t.pairs_per_wave = (int)ceil_div((nb + 1) / 2, std::max(1, t.kwaves));

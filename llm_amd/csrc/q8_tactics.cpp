@@ -179,14 +179,18 @@ void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
 
 // A q, k, v group with its rotation in the epilogue: the plain group's K split
 // (the results are its bits), one token tile a wave.  The epilogue is long and a
-// wave of two token tiles runs it twice in a row (6912 x 2304: n = 512 34.0 us
-// against 32.1, n = 1000 59.5 against 53.4).  From 128 row tiles up two token-tile
-// waves share a workgroup and its weight loads where the token tiles pair off (in
-// a layer at n = 43 0.6 us less; 3 us more where one wave idles, n = 257), up to
-// the workgroup's 16 waves (the rule splits K over eight at most, an option over more).
-void q8_gemm_rope_shape(int n, int out, q8_tactic *t) {
+// wave of two token tiles runs it twice in a row (6912 x 2304 in a layer: n = 576
+// 9 us more, n = 1000 7 more); only on long rows past twenty tiles a CU are the
+// shared weight loads worth as much (12288 x 4096 n = 507 88.9 -> 75.7, n = 1000 172 ->
+// 146; in a layer 1 and 16 us less).  From 128 row tiles up two token-tile waves
+// share a workgroup and its weight loads where the token tiles pair off (in a
+// layer at n = 43 0.6 us less; 3 us more where one wave idles, n = 257), up to the
+// workgroup's 16 waves (the rule splits K over eight at most, an option over more).
+void q8_gemm_rope_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
+    const int rtiles = ceil_div(out, 32), ttiles = ceil_div(n, 32);
+    if (t->tpw == 2 && k >= 40 * 64 && (long long)rtiles * ttiles > 20LL * std::max(cu_count, 1)) return;
     t->tpw = 1;
-    t->twaves = (ceil_div(out, 32) >= 128 && ceil_div(n, 32) % 2 == 0 && t->kwaves <= 8) ? 2 : 1;
+    t->twaves = (rtiles >= 128 && ttiles % 2 == 0 && t->kwaves <= 8) ? 2 : 1;
 }
 
 // The fused gate/up launch (one wave a gate tile, its up tile and one token

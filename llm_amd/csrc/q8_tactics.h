@@ -28,7 +28,7 @@ int q8_tactics_choose(int n, int out, int k, int cu_count, q8_tactic *t);
 // Launch shapes (slots = member tiles per GEMV workgroup: 2 for fused gate/up).
 void q8_gemv_shape(int out, int k, int cu_count, int slots, q8_tactic *t);
 void q8_gemm_shape(int n, int out, int k, int cu_count, q8_tactic *t);
-void q8_gemm_rope_shape(int n, int out, q8_tactic *t);
+void q8_gemm_rope_shape(int n, int out, int k, int cu_count, q8_tactic *t);
 int q8_gemm_silu_kwaves(int n, int ffn, int k, int cu_count);
 void q8_gemm_h_shape(int n, int out, int k, int cu_count, q8_tactic *t);
 /* Staged GEMM launch shape (RW, KW, TPW) for f16 (i8 = 0) or int8 (i8 = 1) activation units. */

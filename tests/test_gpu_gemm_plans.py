@@ -93,7 +93,8 @@ def test_every_tile_has_its_workgroup(gpu, option, tiles):
     (33, 24, 24, 64, 1536, 9), (64, 32, 16, 64, 1536, 0),   # 144 and 128 row tiles, paired: 1024 threads
     (64, 30, 15, 64, 1536, 3), (65, 24, 24, 64, 1536, 3),   # 120 row tiles; three token tiles: unpaired
     (250, 36, 36, 16, 1152, 1), (290, 36, 36, 64, 1152, 0), (256, 9, 3, 0, 576, 40),
-    (96, 24, 24, 64, 224, 2), (64, 24, 24, 64, 32, 7)]] +    # short rows: no K split
+    (96, 24, 24, 64, 224, 2), (64, 24, 24, 64, 32, 7),       # short rows: no K split
+    (416, 64, 64, 64, 2560, 3), (420, 64, 64, 48, 2560, 0)]] +  # 4992 and 5376 tiles: one and two token tiles a wave
     [(64, 24, 24, 64, 1536, 0, 16)])                       # K over all of a workgroup's waves: unpaired
 def test_rotated_group_equals_the_plain_one(gpu, n, heads, kv, n_rot, e, position, kwaves):
     r = np.random.default_rng(SEED + n + heads + kv + e)
