@@ -194,16 +194,22 @@ void q8_gemm_rope_shape(int n, int out, int k, int cu_count, q8_tactic *t) {
 }
 
 // The fused gate/up launch (one wave a gate tile, its up tile and one token
-// tile): as above, four K waves at most (eight were slower at every shape but
-// the smallest K = 2304 ones, by up to 2%), at most 2500 waves.  Over widths
-// 960 .. 5760, K 512 .. 2304 and n 4 .. 1000: within 1.4% of the best on the
-// geometric mean, 12% before (11 waves per CU, nine pairs a wave); 2432 x 896
-// n = 43 10.5 -> 7.0 us, 5760 x 2304 n = 349 44.5 -> 40.4.
+// tile).  Four K waves while 2500 of them are enough for it, two up to six tiles
+// a CU (fewer pairs and a reduction beat a wave of the whole row: 2304 x 1536 n = 550
+// 20.9 -> 18.6 us).  Long rows (80 pairs) take four up to five tiles a CU (4096 x 5760
+// n = 191 37.4 -> 32.4) and eight up to half a tile (256 x 5120 n = 257 13.6 -> 12.1);
+// eight were slower elsewhere.  Over widths 256 .. 8192, K 512 .. 8192 and n 2 .. 1024
+// (460 shapes) within 1.3% of the best on the geometric mean; four and two waves up
+// to 2.4 and 4.9 tiles alone 2.2%, 11 waves per CU with nine pairs a wave 13%.
 int q8_gemm_silu_kwaves(int n, int ffn, int k, int cu_count) {
     const int npairs = ceil_div(k / 32, 2);
     const long long base = (long long)ceil_div(ffn, 32) * ceil_div(n, 32);
-    int kw = npairs < 8 ? 1 : 4;
-    while (kw > 1 && (base * kw * 256 > 2500LL * std::max(cu_count, 1) || npairs < 2 * kw)) kw /= 2;
+    const long long cus = std::max(cu_count, 1);
+    const bool lng = npairs >= 80;
+    int kw = npairs < 8 ? 1 : lng && 2 * base <= cus ? 8 : 4;
+    if (kw == 4 && (lng ? base > 5 * cus : base * 4 * 256 > 2500 * cus)) kw = 2;
+    if (kw == 2 && base > 6 * cus) kw = 1;
+    while (kw > 1 && npairs < 2 * kw) kw /= 2;
     return kw;
 }
 

@@ -128,7 +128,11 @@ def test_rotated_group_equals_the_plain_one(gpu, n, heads, kv, n_rot, e, positio
 
 # (n, ffn, k, K waves)
 @pytest.mark.parametrize("n,ffn,k,kwaves", [(64, 96, 224, 1), (33, 96, 512, 4), (128, 4992, 2304, 4),
-                                            (129, 4032, 2304, 2), (250, 4992, 1056, 2), (257, 4480, 1056, 1)])
+                                            (129, 4032, 2304, 2), (250, 4992, 1056, 2), (257, 4480, 1056, 2),
+                                            (250, 6144, 1056, 2), (250, 6176, 1056, 1),  # six tiles a CU
+                                            # 80 pairs: half a tile and five tiles a CU
+                                            (64, 2048, 5120, 8), (64, 2080, 5120, 4), (64, 2048, 5056, 4),
+                                            (250, 5120, 5120, 4), (250, 5152, 5120, 2)])
 def test_gate_up_on_both_sides_of_the_lines(gpu, n, ffn, k, kwaves):
     r = np.random.default_rng(SEED + n + ffn + k)
     g, u = q8w(r, ffn, k), q8w(r, ffn, k)
