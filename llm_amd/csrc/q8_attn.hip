@@ -367,13 +367,20 @@ extern "C" __global__ __launch_bounds__(512) void q8_attn_decode_w8(Q8_ATTN_PARA
 // MFMA operand sits in lane-half k / 8, slot k % 8, for A and B alike; D[m][n]
 // has n = lane % 32, m = 8(v/4) + 4(lane/32) + v%4.
 //
-// The softmax runs in base 2: q is multiplied by scale log2(e) with its power
-// of two taken out (Q8AttnPrefillArgs), before the split that rounds it to 22
-// bits anyway, so a weight is one fma and one v_exp_f32, with one rounding of
-// the exponent's argument.  A row's reference m moves only when its tile max
-// passes it by more than 8 (weights stay below 2^8, sums in f32), so the
-// accumulators are rescaled in few tiles; it starts finite, so that a row with
-// no visible key yet subtracts no infinity.
+// The softmax runs in base 2: q is multiplied by the fraction of scale log2(e)
+// and the scores by a power of two (exact, so a row's maximum is the bits of one
+// of its scores' products), and a weight is one fma and one v_exp_f32, with one
+// rounding of the exponent's argument.  The query's own power of two goes the same
+// way: its largest element is brought to 2^13 .. 2^14 before the split, where lo
+// stays clear of the f16 subnormals for every element that counts.  Split at the
+// query's own size the error was 2^-25 for elements below 1/4, and 1.4 times that
+// behind the factor of scale 0.125: against 64 bits, queries of 0.01 on keys of 100
+// 2.4e-6 (1.7e-6 without the factor, 2.2e-7 now), of 1 on 1 2.2e-7 as now.  The
+// maximum costs a launch of few keys 2%.
+// A row's reference m moves only when its tile max passes it by more than 8
+// (weights stay below 2^8, sums in f32), so the accumulators are rescaled in few
+// tiles; it starts finite, so that a row with no visible key yet subtracts no
+// infinity.
 // Heavier (later) query tiles of a head are launched first, and the workgroups
 // of a head run on one XCD (round-robin dispatch), whose L2 then serves the
 // head's cache rows to all of them.
@@ -394,8 +401,28 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) const uint8_t lds_bytes_t;
 typedef __attribute__((address_space(3))) void attn_lds_t;
 
-// x as f16 hi + lo, two values an instruction where there is one; the
-// remainder x - hi by one mixed-precision fma (exact), two values of hi a register.
+// c x as f16 hi + lo, two values an instruction where there is one; the remainder
+// c x - hi by one mixed-precision fma, two values of hi a register, so that both
+// parts are of the same hi.
+static __device__ __forceinline__ void split_f16(const float *x, float c, f16x8 &hi, f16x8 &lo) {
+    union Parts {
+        unsigned w[4];
+        f16x8 v;
+    } hp, lp;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        hp.w[i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){x[2 * i] * c, x[2 * i + 1] * c}, f16x2));
+        float l0, l1;
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(l0) : "v"(x[2 * i]), "v"(c), "v"(hp.w[i]));
+        asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+            : "=v"(l1)
+            : "v"(x[2 * i + 1]), "v"(c), "v"(hp.w[i]));
+        lp.w[i] = __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2){l0, l1}, f16x2));
+    }
+    hi = hp.v;
+    lo = lp.v;
+}
+// The same of x itself.
 static __device__ __forceinline__ void split_f16(const float *x, f16x8 &hi, f16x8 &lo) {
     union Parts {
         unsigned w[4];
@@ -510,16 +537,28 @@ static __device__ __forceinline__ void attn_prefill_body(const Q8AttnPrefillArgs
         __builtin_amdgcn_sched_barrier(0);
         load_tile(khead, kg, kbuf);
         load_tile(vhead, kg, vbuf);
-        // Q^T operand, d-step s: q[qrow][16s + 8h .. +7] as f16 hi/lo
+        // Q^T operand, d-step s: q[qrow][16s + 8h .. +7] times q_mult and the row's
+        // power of two, as f16 hi/lo; lo from the unrounded product
+        float top_q = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                if (!qlive) qv[s][i] = 0.0f;
+                top_q = fmaxf(top_q, fabsf(qv[s][i]));
+            }
+        top_q = xor_max<32>(top_q);
+        const int qe = max(__builtin_amdgcn_frexp_expf(top_q), -100);  // 0 for 0; the power stays finite
+        const float qm = __builtin_ldexpf(a.q_mult, 14 - qe);
+        const float s2 = __builtin_ldexpf(1.0f, min(max(a.s_exp + qe - 14, -126), 127));
         f16x8 qhi[4], qlo[4];
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             float x[8];
 #pragma unroll
-            for (int i = 0; i < 8; i++) x[i] = qlive ? qv[2 * s + (i >> 2)][i & 3] * a.q_mult : 0.0f;
-            split_f16(x, qhi[s], qlo[s]);
+            for (int i = 0; i < 8; i++) x[i] = qv[2 * s + (i >> 2)][i & 3];
+            split_f16(x, qm, qhi[s], qlo[s]);
         }
-        const float s2 = a.s_mult;
         const int lim = min(qa, kend - 1);  // last key this lane's query sees
         int koff[4];
 #pragma unroll

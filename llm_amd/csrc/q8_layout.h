@@ -330,7 +330,8 @@ typedef struct {
     float *out;             /* [n][n_head][head_dim], or null */
     const int *position;    /* device: cache position of query 0 */
     int n, n_head, n_kv, capacity, qtiles;
-    float q_mult, s_mult;   /* scale log2(e) = q_mult s_mult: q_mult in [1/2, 1) (or +-0), s_mult a power of two */
+    float q_mult;           /* scale log2(e) = q_mult 2^s_exp: q_mult in [1/2, 1] (or its negative, or 0) */
+    int s_exp;
     uint8_t *xq;            /* non-null: the output also as prepared Q8_0 (units, as q8_quantize writes them) */
     float *xs;              /* its block scales */
     int f16;                /* 1: f16 prepared units */

@@ -2567,9 +2567,7 @@ int run_attn_prefill(q8_ctx *c, const float *q, q8_dptr kcache, q8_dptr vcache, 
     a.n_kv = n_kv;
     a.capacity = capacity;
     a.qtiles = (int)ceil_div(n, 32);
-    int e2 = 0;
-    a.q_mult = (float)std::frexp((double)scale * 1.4426950408889634, &e2);
-    a.s_mult = (float)std::ldexp(1.0, e2);
+    a.q_mult = (float)std::frexp((double)scale * 1.4426950408889634, &a.s_exp);
     if (p) {
         const int k = n_head * Q8_ATTN_HEAD_DIM;
         const int nb = k / 32;

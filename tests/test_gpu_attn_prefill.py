@@ -77,3 +77,79 @@ def test_rows_past_the_context_are_not_read(gpu):
     assert np.abs(got - ref).max() <= 5e-6
     for b in (qb, out, kc, vc, pos):
         b.free()
+
+
+@pytest.mark.parametrize("scale", [0.125, 0.09, -0.125, 0.36])
+@pytest.mark.parametrize("n,start,heads", [(40, 30, 3), (290, 10, 29)])
+def test_small_queries_against_large_keys(gpu, n, start, heads, scale):
+    """A query's two f16 parts carry 22 bits of each element at any size: the bar
+    above, with elements of 2^-16 and keys of 2^15.  Split at its own size such an element's
+    second part is an f16 subnormal, rounded at 2^-25, which is 2^-10 of a key."""
+    r = np.random.default_rng(SEED + n)
+    capacity = start + n
+    kf = (r.uniform(-1, 1, (capacity, heads, 64)) * 32000).astype(np.float16).astype(np.float32)
+    vf = r.standard_normal((capacity, heads, 64)).astype(np.float16).astype(np.float32)
+    q = (r.integers(-255, 256, (n, heads, 64)) * 2.0 ** -24).astype(np.float32)
+    kc, vc, qb, out = gpu.alloc(2 * kf.size), gpu.alloc(2 * vf.size), gpu.alloc(q.nbytes), gpu.alloc(q.nbytes)
+    kc.upload(kf.astype(np.float16))
+    vc.upload(vf.astype(np.float16))
+    qb.upload(q)
+    pos = int_buffer(gpu, start)
+    print(f"\nsmall queries n={n} heads={heads} scale={scale}", flush=True)
+    gpu.attention(qb, kc, vc, out, n, heads, heads, 64, capacity, scale, pos)
+    got = out.download(np.float32, q.size).reshape(q.shape)
+    ref = oracle.attention(q, kf, vf, start, scale)
+    size = max((np.abs(q[:, h]).astype(np.float64) @ np.abs(kf[:, h]).T.astype(np.float64)).max() for h in range(heads))
+    delta = 2.0 ** -21 * size * abs(scale)
+    bar = 2 * delta * np.abs(vf).max() + 2e-6 + 1e-5 * np.abs(ref)
+    worst = (np.abs(got - ref) / bar).max()
+    assert worst <= 1, f"{worst:.2f} of the bar"
+    for b in (qb, out, kc, vc, pos):
+        b.free()
+
+
+# (scale, query std): scores near 8 std^2 scale
+@pytest.mark.parametrize("scale,std", [(3e38, 1e-3), (-3.4e38, 1e-3)])
+@pytest.mark.parametrize("n,heads", [(40, 2), (290, 29)])
+def test_scores_far_apart_pick_one_key(gpu, n, heads, scale, std):
+    """At such scales every query's weights are one 1 and zeros: the output is its best key's
+    value, exactly, also where all the scores that a query sees are far below zero."""
+    r = np.random.default_rng(SEED + n)
+    kf, vf, kc, vc = cache_pair(gpu, r, n, n, heads)
+    q = (r.standard_normal((n, heads, 64)) * std).astype(np.float32)
+    qb, out, pos = gpu.alloc(q.nbytes), gpu.alloc(q.nbytes), int_buffer(gpu, 0)
+    qb.upload(q)
+    print(f"\nscale {scale} n={n} heads={heads}", flush=True)
+    gpu.attention(qb, kc, vc, out, n, heads, heads, 64, n, scale, pos)
+    got = out.download(np.float32, q.size).reshape(q.shape)
+    checked = 0
+    for h in range(heads):
+        s = (q[:, h].astype(np.float64) @ kf[:, h].T.astype(np.float64)) * np.sign(scale)
+        s[np.triu_indices(n, 1)] = -np.inf
+        top = np.sort(s, axis=1)
+        # two f16 parts of q and a f32 sum: the order of scores further apart than this is certain
+        apart = np.full(n, True)
+        apart[1:] = top[1:, -1] - top[1:, -2] > 2.0 ** -18 * np.abs(q[1:, h]).max() * 64 * np.abs(kf[:, h]).max()
+        want = vf[s.argmax(1), h]
+        assert np.array_equal(got[apart, h], want[apart]), f"head {h}"
+        checked += int(apart.sum())
+    assert checked >= 0.95 * n * heads
+    for b in (qb, out, kc, vc, pos):
+        b.free()
+
+
+def test_zero_scale_averages(gpu):
+    """Scale 0 and the least subnormal weigh every visible key alike."""
+    n, heads = 45, 2
+    r = np.random.default_rng(SEED)
+    kf, vf, kc, vc = cache_pair(gpu, r, n, n, heads)
+    q = r.standard_normal((n, heads, 64)).astype(np.float32)
+    qb, out, pos = gpu.alloc(q.nbytes), gpu.alloc(q.nbytes), int_buffer(gpu, 0)
+    qb.upload(q)
+    for scale in (0.0, -0.0, 1e-45, -1e-45):
+        gpu.attention(qb, kc, vc, out, n, heads, heads, 64, n, scale, pos)
+        got = out.download(np.float32, q.size).reshape(q.shape)
+        ref = oracle.attention(q, kf, vf, 0, scale)
+        assert np.abs(got - ref).max() <= 5e-6, scale
+    for b in (qb, out, kc, vc, pos):
+        b.free()
