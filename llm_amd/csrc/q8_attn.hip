@@ -524,7 +524,7 @@ static __device__ __forceinline__ void attn_prefill_body(const Q8AttnPrefillArgs
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    float m = -3e38f, l = 0.0f;  // below any score; l: this lane's half of the keys
+    float m = -FLT_MAX, l = 0.0f;  // not above any finite score; l: this lane's half of the keys
     f32x16 o[2] = {};
     if (kg < groups) {
         // q's loads first (they need no position), then the first tile's

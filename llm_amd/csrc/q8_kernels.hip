@@ -21,6 +21,7 @@
 //                                                              (gpu.cu rmsnorm_rows, rmsnorm_quantize_rows 351-407)
 #include <hip/hip_runtime.h>
 
+#include <cfloat>
 #include <type_traits>
 
 #include "q8_layout.h"

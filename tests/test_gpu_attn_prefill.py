@@ -109,7 +109,8 @@ def test_small_queries_against_large_keys(gpu, n, start, heads, scale):
 
 
 # (scale, query std): scores near 8 std^2 scale
-@pytest.mark.parametrize("scale,std", [(3e38, 1e-3), (-3.4e38, 1e-3)])
+@pytest.mark.parametrize("scale,std", [(1e20, 1), (-1e20, 1), (1e30, 1), (-1e30, 1), (1e36, 1), (3e38, 1e-3),
+                                       (-3.4e38, 1e-3)])
 @pytest.mark.parametrize("n,heads", [(40, 2), (290, 29)])
 def test_scores_far_apart_pick_one_key(gpu, n, heads, scale, std):
     """At such scales every query's weights are one 1 and zeros: the output is its best key's
@@ -138,6 +139,23 @@ def test_scores_far_apart_pick_one_key(gpu, n, heads, scale, std):
         b.free()
 
 
+def test_scores_near_the_end_of_the_range(gpu):
+    """All of a row's scores at -2.2e38, -3.2e38 in units of log2: equal, so its keys weigh alike."""
+    n, heads = 40, 2
+    r = np.random.default_rng(SEED)
+    kf, vf, kc, vc = cache_pair(gpu, r, n, n, heads)
+    kc.upload(np.full(n * heads * 64, 1.25, np.float16))
+    q = np.full((n, heads, 64), 1.25, np.float32)
+    qb, out, pos = gpu.alloc(q.nbytes), gpu.alloc(q.nbytes), int_buffer(gpu, 0)
+    qb.upload(q)
+    gpu.attention(qb, kc, vc, out, n, heads, heads, 64, n, -2.22e36, pos)
+    got = out.download(np.float32, q.size).reshape(q.shape)
+    want = np.cumsum(vf.astype(np.float64), axis=0) / np.arange(1, n + 1)[:, None, None]
+    assert np.abs(got - want).max() <= 5e-6
+    for b in (qb, out, kc, vc, pos):
+        b.free()
+
+
 def test_zero_scale_averages(gpu):
     """Scale 0 and the least subnormal weigh every visible key alike."""
     n, heads = 45, 2
@@ -151,5 +169,24 @@ def test_zero_scale_averages(gpu):
         got = out.download(np.float32, q.size).reshape(q.shape)
         ref = oracle.attention(q, kf, vf, 0, scale)
         assert np.abs(got - ref).max() <= 5e-6, scale
+    for b in (qb, out, kc, vc, pos):
+        b.free()
+
+
+def test_a_nan_key_reaches_the_queries_that_see_it(gpu):
+    """A score that is no number makes its query's output no number (the reference's softmax
+    sums it) and leaves the queries before it, in the same tile, as they were."""
+    n, heads, at = 70, 2, 41
+    r = np.random.default_rng(SEED)
+    kf, vf, kc, vc = cache_pair(gpu, r, n, n, heads)
+    q = r.standard_normal((n, heads, 64)).astype(np.float32)
+    ref = oracle.attention(q, kf, vf, 0, 0.125)
+    kc.upload(np.full(heads * 64, np.nan, np.float16), at * heads * 64 * 2)
+    qb, out, pos = gpu.alloc(q.nbytes), gpu.alloc(q.nbytes), int_buffer(gpu, 0)
+    qb.upload(q)
+    gpu.attention(qb, kc, vc, out, n, heads, heads, 64, n, 0.125, pos)
+    got = out.download(np.float32, q.size).reshape(q.shape)
+    assert np.abs(got[:at] - ref[:at]).max() <= 5e-6
+    assert np.isnan(got[at:]).all()
     for b in (qb, out, kc, vc, pos):
         b.free()
