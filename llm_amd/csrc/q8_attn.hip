@@ -703,8 +703,8 @@ static __device__ __forceinline__ void attn_prefill_body(const Q8AttnPrefillArgs
     }
 }
 
-// Four waves a workgroup (four workgroups a CU), or eight where there are too
-// few workgroups to fill the chip with four (run_attn_prefill).
+// Four waves a workgroup, or eight while every workgroup has a CU to itself
+// (run_attn_prefill has the times).
 extern "C" __global__ __launch_bounds__(256, 4) void q8_attn_prefill(Q8AttnPrefillArgs a) { attn_prefill_body<4>(a); }
 extern "C" __global__ __launch_bounds__(512, 4) void q8_attn_prefill_k8(Q8AttnPrefillArgs a) {
     attn_prefill_body<8>(a);
