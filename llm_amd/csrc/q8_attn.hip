@@ -375,8 +375,7 @@ extern "C" __global__ __launch_bounds__(512) void q8_attn_decode_w8(Q8_ATTN_PARA
 // stays clear of the f16 subnormals for every element that counts.  Split at the
 // query's own size the error was 2^-25 for elements below 1/4, and 1.4 times that
 // behind the factor of scale 0.125: against 64 bits, queries of 0.01 on keys of 100
-// 2.4e-6 (1.7e-6 without the factor, 2.2e-7 now), of 1 on 1 2.2e-7 as now.  The
-// maximum costs a launch of few keys 2%.
+// 2.4e-6 (1.7e-6 without the factor, 2.2e-7 now), of 1 on 1 2.2e-7 as now.
 // A row's reference m moves only when its tile max passes it by more than 8
 // (weights stay below 2^8, sums in f32), so the accumulators are rescaled in few
 // tiles; it starts finite, so that a row with no visible key yet subtracts no
@@ -538,15 +537,13 @@ static __device__ __forceinline__ void attn_prefill_body(const Q8AttnPrefillArgs
         load_tile(khead, kg, kbuf);
         load_tile(vhead, kg, vbuf);
         // Q^T operand, d-step s: q[qrow][16s + 8h .. +7] times q_mult and the row's
-        // power of two, as f16 hi/lo; lo from the unrounded product
+        // power of two, as f16 hi/lo; lo from the unrounded product (the last tile's
+        // padding queries repeat the last one: their outputs are cleared at the end)
         float top_q = 0.0f;
 #pragma unroll
         for (int s = 0; s < 8; s++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                if (!qlive) qv[s][i] = 0.0f;
-                top_q = fmaxf(top_q, fabsf(qv[s][i]));
-            }
+            for (int i = 0; i < 4; i++) top_q = fmaxf(top_q, fabsf(qv[s][i]));
         top_q = xor_max<32>(top_q);
         const int qe = max(__builtin_amdgcn_frexp_expf(top_q), -100);  // 0 for 0; the power stays finite
         const float qm = __builtin_ldexpf(a.q_mult, 14 - qe);
